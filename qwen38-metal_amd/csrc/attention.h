@@ -13,6 +13,11 @@ constexpr int kMaxPagesPerSplit = 1024;  // pages per decode workgroup
 // the next kernel width, the extra dimensions are zero.
 inline uint32_t attn_padded_dim(uint32_t d) { return d <= 64 ? 64 : d <= 128 ? 128 : 256; }
 
+// Waves per SIMD that the prefill kernel's registers are cut for at storage
+// dimension D and W waves a workgroup: the O^T accumulators take D / 2 and the
+// Q operand D / 4.
+constexpr int attn_prefill_waves(uint32_t D, int W) { return D == 64 ? 3 : D == 256 && W == 4 ? 1 : 2; }
+
 struct AttnSeq {
   int8_t* k;          // K pages   [page][kv_head][16][D]
   int8_t* v;          // V pages   [page][kv_head][D][16]
@@ -43,19 +48,20 @@ struct AttnArgs {
   const uint16_t* q;     // bf16 [rows][H][D]
   const uint16_t* gate;  // bf16 [rows][H][D] or null
   uint16_t* o;           // bf16 [rows][H][D]
-  float* partials;       // decode split partials: O [split rows][H][Dp], then (m, l) [split rows][H][2]
+  float* partials;       // split partials: O [split rows][H][Dp], then (m, l) [split rows][H][2]
   const float* k_new;    // decode: fp32 [n_seqs][kv_heads][D] rows appended by the kernel
   const float* v_new;
   uint32_t heads;
   uint32_t kv_heads;
   uint32_t head_dim;      // real head dimension (strides of q, gate, o, k_new, v_new)
   uint32_t head_dim_pad;  // storage dimension Dp of the cache pages (64, 128 or 256)
-  uint32_t part_rows;     // decode: split rows in `partials` (offset of the (m, l) table)
+  uint32_t part_rows;     // split rows in `partials` (offset of the (m, l) table)
   uint32_t n_seqs;
   uint32_t pages_per_split;  // decode
-  uint32_t wg_waves;         // decode: waves per workgroup (4: two workgroups per CU; 8: one)
-  int32_t prefill_cb;        // prefill: column blocks per wave (0: the default for D)
+  uint32_t wg_waves;         // waves per workgroup, 4 or 8 (decode: two workgroups per CU, or one)
   uint32_t prefill;
+  uint32_t splits;           // prefill: workgroups sharing the tiles of a column block
+  uint32_t out8;             // prefill: o and gate rows take 8-byte accesses
   uint32_t rows;   // prefill: query rows
   uint32_t start;  // prefill: cache position of row 0
   AttnSeq seqs[kMaxAttnSeqs];

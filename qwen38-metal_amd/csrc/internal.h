@@ -63,7 +63,8 @@ struct Tuning {
   int attn_pps = 0;         // QM38_ATTN_PPS: pages per decode split
   int attn_waves = 0;       // QM38_ATTN_WAVES: 4 or 8 waves per decode workgroup
   int attn_target_wgs = 0;  // QM38_ATTN_TARGET_WGS
-  int prefill_cb = 0;       // QM38_PREFILL_CB: column blocks per prefill wave (1, 2, 4)
+  int prefill_splits = 0;   // QM38_PREFILL_SPLITS: workgroups sharing a prefill column block's tiles
+  int prefill_waves = 0;    // QM38_PREFILL_WAVES: 4 or 8 waves per prefill workgroup
   int dn_step_head = -1;    // QM38_DN_STEP_HEAD: 0 forces the split step kernel (-1: default)
   int dn_chunked = -1;      // QM38_DN_CHUNKED: 1 / 0 forces the chunked / token-serial prefill (-1: default)
   int dn_pair = -1;         // QM38_DN_PAIR: 0 forces the one-value-head chunk preparation (-1: default)

@@ -12,9 +12,10 @@
 //    and round-half-away-from-zero, and writes page-table entries of pages
 //    materialised by this append.
 //  * q8_prefill_kernel (causal prefill) and q8_decode_kernel (decode):
-//    flash attention over Q8 pages.  A wave owns one KV head and the GQA group
-//    of <= 16 query heads sharing it (decode), or CB blocks of 16 (row, head)
-//    columns (prefill).  Per 16-token page:
+//    flash attention over Q8 pages.  A decode wave owns one KV head and the GQA
+//    group of <= 16 query heads sharing it; a prefill wave 32 (row, head)
+//    columns of one KV head (its structure is described at the kernel).  Per
+//    16-token page of decode:
 //      S^T = K Q^T on fp16 MFMA 16x16x32 (K bytes -> fp16 of 1024 + (k + 128)
 //      exactly, one AND-OR per pair; 1152 * sum(q) is removed per column),
 //      online softmax in fp32 (exp2 domain, lazy rescaling),
@@ -253,6 +254,12 @@ __device__ __forceinline__ u32x2 q8x4_to_f16_biased(uint32_t w) {
   const uint32_t u = w ^ 0x80808080u;
   return u32x2{(u & 0x00FF00FFu) | 0x64006400u, ((u >> 8) & 0x00FF00FFu) | 0x64006400u};
 }
+// The same as signed values: minus 1152, exact in fp16.
+__device__ __forceinline__ u32x2 q8x4_to_f16_signed(uint32_t w) {
+  typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+  const half4_t bias = {(_Float16)1152.0f, (_Float16)1152.0f, (_Float16)1152.0f, (_Float16)1152.0f};
+  return __builtin_bit_cast(u32x2, __builtin_bit_cast(half4_t, q8x4_to_f16_biased(w)) - bias);
+}
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 // 4 signed int8 -> bf16 pairs (b0, b1), (b2, b3), exact (v_cvt_f32_i32 with a
 // sign-extended byte select, then v_cvt_pk_bf16_f32).
@@ -274,6 +281,16 @@ __device__ __forceinline__ float max4_across_kq(float v) {
   const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+__device__ __forceinline__ floatx16 mfma32x32x16_f16(u32x4 a, u32x4 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0,
+                                                0, 0);
+}
+// Maximum over lanes l and l ^ 32 (the two halves of one 32-wide MFMA column).
+__device__ __forceinline__ float max2_across_halves(float v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
 
 template <bool B>
@@ -635,12 +652,13 @@ __global__ __launch_bounds__(256) void q8_combine_kernel(AttnArgs args) {
   const uint32_t wq = blockIdx.x % kWgPerHead;
   const uint32_t bh = blockIdx.x / kWgPerHead;
   const uint32_t b = bh / H, hh = bh % H;
-  const AttnSeq& sq = args.seqs[b];
-  const uint32_t ns = sq.nsplit;
+  // b is a sequence (decode) or a query row (prefill: the same splits for all).
+  const uint32_t ns = args.prefill ? args.splits : args.seqs[b].nsplit;
   if (ns <= 1 || 32 * wq >= dr) return;
+  const size_t part_begin = args.prefill ? (size_t)b * ns : args.seqs[b].part_begin;
   const size_t o_rows = (size_t)args.part_rows * H;
-  const float* obase = args.partials + ((size_t)sq.part_begin * H + hh) * D;
-  const float* mbase = args.partials + o_rows * D + ((size_t)sq.part_begin * H + hh) * 2;
+  const float* obase = args.partials + (part_begin * H + hh) * D;
+  const float* mbase = args.partials + o_rows * D + (part_begin * H + hh) * 2;
   const uint32_t t = threadIdx.x, c = t % 8, g = t / 8;
   const uint32_t d0 = 32 * wq + 4 * c;
 
@@ -718,12 +736,13 @@ __global__ __launch_bounds__(64) void q8_combine_small_kernel(AttnArgs args) {
   const uint32_t wq = blockIdx.x % kWgPerHead;
   const uint32_t bh = blockIdx.x / kWgPerHead;
   const uint32_t b = bh / H, hh = bh % H;
-  const AttnSeq& sq = args.seqs[b];
-  const uint32_t ns = sq.nsplit;
+  // b is a sequence (decode) or a query row (prefill: the same splits for all).
+  const uint32_t ns = args.prefill ? args.splits : args.seqs[b].nsplit;
   if (ns <= 1 || 32 * wq >= dr) return;
+  const size_t part_begin = args.prefill ? (size_t)b * ns : args.seqs[b].part_begin;
   const size_t o_rows = (size_t)args.part_rows * H;
-  const float* obase = args.partials + ((size_t)sq.part_begin * H + hh) * D;
-  const float* mbase = args.partials + o_rows * D + ((size_t)sq.part_begin * H + hh) * 2;
+  const float* obase = args.partials + (part_begin * H + hh) * D;
+  const float* mbase = args.partials + o_rows * D + (part_begin * H + hh) * 2;
   const uint32_t t = threadIdx.x, c = t % 8, g = t / 8;
   const uint32_t d0 = 32 * wq + 4 * c;
   floatx4 ov[kPer];
@@ -772,313 +791,458 @@ __global__ __launch_bounds__(64) void q8_combine_small_kernel(AttnArgs args) {
   }
 }
 
-// Causal prefill: blockIdx.x = rb * KVH + kvh.  A wave owns CB column
-// blocks of 16 (row, head) columns, i.e. CB * 16 / gh query rows of one KV
-// head; the workgroup's four waves own consecutive rows and walk the same
-// pages, which are unpacked once per workgroup into LDS (each wave a
-// quarter) and serve every wave's CB blocks.
-template <int D, int CB>
-__global__ __launch_bounds__(256) void q8_prefill_kernel(AttnArgs args) {
-  constexpr int kWaves = 4;
-  constexpr int kDB = D / 16;  // 16-wide d blocks of O^T
-  constexpr int kKS = D / 32;  // QK k-steps
+// Four outputs as bf16, and with the sigmoid of four bf16 gates.  The gate
+// takes v_exp_f32 and v_rcp_f32 (within an ulp each; the error of the product
+// -v log2(e) grows with |v| and stays below 2^-16 of the result for every gate
+// whose sigmoid is above 1e-30, against the 2^-9 of the bf16 store): the
+// library forms took longer than a tile's softmax.
+__device__ __forceinline__ u32x2 bf16x4_of(floatx4 v) {
+  return u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
+               (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
+}
+__device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = i < 2 ? gate.x : gate.y;
+    const float x = i & 1 ? bf16_hi_f32(w) : bf16_lo_f32(w);
+    v[i] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * x));
+  }
+  return bf16x4_of(v);
+}
+
+// Causal prefill on 32x32x16 MFMA.  The rows of one KV head are a list of
+// columns, column c = (row c / gh, query head c % gh of the group), so every
+// lane of a 32-wide MFMA column block has work whatever the group size.  A
+// workgroup owns 32 W consecutive columns (32 per wave) and one range of the
+// 32-token tiles (two pages) that its last row sees; a tile is unpacked once
+// per workgroup into LDS and serves every wave:
+//   S^T[token][column] = K Q^T     (fp16; K exactly, as integers)
+//   O^T[d][column]    += V^T P'^T  (bf16; V exactly, P' = p * v_scale as hi + lo)
+// A lane holds 16 of a column's 32 scores and its pair (lane ^ 32) the
+// others, so the softmax needs one exchange per tile, and the scores leave
+// the first product in the order in which the second one's B operand takes
+// them: V's tokens are laid out to match, and P' never crosses lanes.
+//
+// Few rows leave the chip idle if one workgroup walks all tiles (5 rows of
+// 24 / 4 heads on 20001 tokens ran on 4 workgroups, 1570 us), so the tiles
+// are then split over args.splits workgroups, whose (O, m, l) the combine
+// kernel merges (37 us with the merge).
+//
+// What bounds it: at 2048 rows on 4096 tokens (64 / 8 heads of 128) about 220
+// VALU operations and 24 MFMAs (768 cycles) per wave and tile, two waves per
+// SIMD; 505 us, 680 TFLOP/s.  The 16-wide kernel before it (one page a step,
+// columns padded to the group size, the maximum exchanged every page) took
+// 870 us.
+template <int D, int W>
+struct PrefillLds {
+  static constexpr int kK = 32 * D * 2, kV = 32 * D * 2;
+  static constexpr int kStage = kK + kV + 256;  // K fp16, V bf16, 32 K scales, 32 V scales
+  // Steps of the Q operand that wait in LDS: half of them where D = 256 leaves
+  // two waves a SIMD no registers for all.
+  static constexpr int kQSteps = D == 256 && W == 8 ? D / 32 : 0;
+  static constexpr int kBytes = 2 * kStage + W * kQSteps * 1024;
+};
+
+template <int D, int W>
+__global__ __launch_bounds__(64 * W, attn_prefill_waves(D, W)) void q8_prefill_kernel(AttnArgs args) {
+  using L = PrefillLds<D, W>;
+  constexpr int kDB = D / 32;  // 32-wide d blocks of O^T
+  constexpr int kKS = D / 16;  // QK k-steps
+  // K operands in registers at a time, and V operands taken ahead of the softmax.
+  constexpr int kGroup = D == 256 ? 1 : kKS < 8 ? kKS : 8, kAhead = D == 256 ? 0 : kDB;
+  constexpr int kUnits = (4 * D + 64 * W - 1) / (64 * W);  // 16-byte units of a tile per thread
+  __shared__ __attribute__((aligned(16))) uint8_t lds[L::kBytes];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 15;  // (row, head) column within a block
-  const int kq = lane >> 4;
+  const int lc = lane & 31, hf = lane >> 5;
   const uint32_t H = args.heads, KVH = args.kv_heads, gh = H / KVH;  // gh <= 16
-
-  const uint32_t rows_per_block = 16 / gh, rows_per_wave = CB * rows_per_block;
-  const uint32_t row_blocks = (args.rows + rows_per_wave * kWaves - 1) / (rows_per_wave * kWaves);
-  // KV head = blockIdx % KVH: workgroups are dealt round-robin to the 8 XCDs,
-  // so every row block of one KV head runs on the same XCD(s) and its pages
-  // (1.5 MiB per head at 6K tokens, d = 128) stay in that XCD's L2.
-  const uint32_t kvh = blockIdx.x % KVH;
-  // Row blocks are dealt last first: the later rows see the most pages, and
-  // starting the longest workgroups first lets the short ones fill the
-  // slots they free (the grid runs in about two residency rounds).
-  const uint32_t rb = row_blocks - 1 - blockIdx.x / KVH;
-  const uint32_t row_base = (rb * kWaves + wave) * rows_per_wave;
   const AttnSeq& sq = args.seqs[0];
 
-  const uint32_t ch = col % gh, cr = col / gh;
-  const uint32_t head = kvh * gh + ch;
-  bool col_ok[CB];
-  uint32_t qrow[CB], visible[CB];
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    qrow[cb] = row_base + cb * rows_per_block + cr;
-    col_ok[cb] = (uint32_t)col < rows_per_block * gh && qrow[cb] < args.rows;
-    visible[cb] = min(args.start + qrow[cb] + 1, sq.len);
-  }
+  // KV head = blockIdx % KVH: workgroups are dealt round-robin to the 8 XCDs,
+  // so the column blocks of one KV head run on the same XCD(s) and its pages
+  // stay in that XCD's L2.  Column blocks are dealt last first: the later
+  // rows see the most tiles, and the short workgroups fill the slots they free.
+  const uint32_t cols = args.rows * gh;
+  const uint32_t blocks = (cols + 32 * W - 1) / (32 * W);
+  const uint32_t kvh = blockIdx.x % KVH, bs = blockIdx.x / KVH;
+  const uint32_t S = args.splits, split = bs % S, rb = blocks - 1 - bs / S;
+  const uint32_t c0 = rb * 32 * W + wave * 32;
+  // Columns past the last one repeat it and are not stored.
+  const uint32_t c = min(c0 + lc, cols - 1);
+  const bool col_ok = c0 + lc < cols;
+  const uint32_t row = c / gh, head = kvh * gh + (c - row * gh);
+  const uint32_t visible = min(args.start + row + 1, sq.len);
 
-  // Q operands (B of QK^T) in fp16: lane (col, kq) of block cb holds
-  // q[qrow][head][D/4 kq + 8 j .. + 7] in the element order d0,d2,d1,d3,
-  // d4,d6,d5,d7 that the int8 -> fp16 unpack of K produces.  bf16 -> fp16 is
-  // exact within fp16's range.  K enters as 1024 + (k + 128): 1152 * sum(q)
-  // is subtracted from every score.
+  // The tiles of this workgroup: its share of those its last row sees.
+  const uint32_t last_row = (min(cols, (rb + 1) * 32 * W) - 1) / gh;
+  const uint32_t n_tiles = (min(args.start + last_row + 1, sq.len) + 31) / 32;
+  const uint32_t t0 = (uint32_t)((uint64_t)n_tiles * split / S), t1 = (uint32_t)((uint64_t)n_tiles * (split + 1) / S);
+  const uint32_t last_page = (sq.len - 1) / 16;
+
+  // Q operand (B of QK^T) in fp16: lane (column, hf) of step s holds
+  // q[16 s + 8 hf .. + 7] in the element order d0,d2,d1,d3,d4,d6,d5,d7 of the
+  // int8 -> fp16 unpack of K.  bf16 -> fp16 is exact within fp16's range.
   const uint32_t dr = args.head_dim;  // real head dimension; D is the page storage width
   const bool full_d = dr == (uint32_t)D;
-  u32x4 qb[CB][kKS];
-  float qcorr[CB];
+  constexpr int kQReg = kKS - L::kQSteps;
+  u32x4 qb[kQReg];
+  u32x4* ql = (u32x4*)(lds + 2 * L::kStage) + wave * L::kQSteps * 64 + lane;  // read by the lane that wrote it
+  {
+    const uint16_t* qp = args.q + ((size_t)row * H + head) * dr;
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    const uint16_t* qp = args.q + ((size_t)qrow[cb] * H + head) * dr;
-    float qsum = 0.0f;
-#pragma unroll
-    for (int jj = 0; jj < kKS; ++jj) {
-      const u32x4 v = col_ok[cb] ? load_bf16x8(qp, D / 4 * kq + 8 * jj, dr, full_d) : u32x4{0u, 0u, 0u, 0u};
-      float f[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f[2 * e] = bf16_to_f32(v[e] & 0xFFFFu);
-        f[2 * e + 1] = bf16_to_f32(v[e] >> 16);
-      }
+    for (int s = 0; s < kKS; ++s) {
+      const u32x4 v = load_bf16x8(qp, 16 * s + 8 * hf, dr, full_d);
       const int order[8] = {0, 2, 1, 3, 4, 6, 5, 7};
       uint32_t h[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const _Float16 x = (_Float16)f[order[e]];
-        qsum += (float)x;
+        const uint32_t w = v[order[e] >> 1];
+        const _Float16 x = (_Float16)((order[e] & 1) ? bf16_hi_f32(w) : bf16_lo_f32(w));
         h[e] = __builtin_bit_cast(uint16_t, x);
       }
-      qb[cb][jj] = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+      const u32x4 x = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+      if (s < kQReg) qb[s] = x;
+      else ql[64 * (s - kQReg)] = x;
     }
-    qsum += __shfl_xor(qsum, 16);
-    qsum += __shfl_xor(qsum, 32);
-    qcorr[cb] = 1152.0f * qsum;
   }
   const float sm_scale = kLog2e / sqrtf((float)dr);
 
-  floatx4 o[CB][kDB];
-  float m_run[CB], l_lane[CB];
+  floatx16 o[kDB];
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-    for (int i = 0; i < kDB; ++i) o[cb][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    m_run[cb] = -INFINITY;
-    l_lane[cb] = 0.0f;
-  }
+  for (int i = 0; i < kDB; ++i) o[i] = floatx16{};
+  // The lowest finite value: a column that sees nothing of a tile adds
+  // exp2(-inf) = 0.
+  float m_run = -FLT_MAX, l_lane = 0.0f;
 
-  const size_t kv_page_stride = (size_t)KVH * 16 * D;
-  const int tok = lane & 15;  // A-operand row: token of QK^T, d row of PV^T
-
-  // The four waves walk the same pages.  Each page is unpacked once per
-  // workgroup into an LDS stage (each wave a quarter of it) and every wave
-  // reads its MFMA operands from there:
-  //   K: u32x4 unit (j, kq, tok) = fp16 of 1024 + (k + 128) for
-  //      K[tok][D/4 kq + 8 j .. + 7] in the order d0,d2,d1,d3,d4,d6,d5,d7,
-  //      at row j * 4 + kq, slot tok ^ (row & 15);
-  //   V: u32x2 unit (db, kq, d) = bf16 of V^T[16 db + d][4 kq .. 4 kq + 3]
-  //      at row db * 4 + kq, slot d ^ 4 kq;
-  //   scales: K scale * softmax scale, then V scale, per token.
-  // The slot swizzles keep both the unpacking writes and the operand reads
-  // (16 lanes, one row, all slots) free of bank conflicts.
-  constexpr int kKUnits = 16 * D / 8;  // 8-byte units of one page's K (or V)
-  constexpr int kPerLane = (kKUnits / kWaves + 63) / 64;
-  constexpr int kStage = 16 * D * 2 + 16 * D * 2 + 128;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kStage];
-  const int wave_unit0 = wave * (kKUnits / kWaves);
-
-  // Last row of the workgroup bounds every wave's page walk, so all waves
-  // pass the same barriers; pages past a wave's own rows are fully masked.
-  const uint32_t wg_row0 = rb * kWaves * rows_per_wave;
-  const uint32_t wg_last = min(args.rows, wg_row0 + kWaves * rows_per_wave) - 1;
-  const uint32_t n_pages = (min(args.start + wg_last + 1, sq.len) + 15) / 16;
-
+  // A tile's 4 D 16-byte units: K of its two pages, then V (D units a page).
+  // Unit u of a K page holds token u / (D / 16), d 16 (u % (D / 16)) .. + 15;
+  // unit u of a V page holds d = u, its 16 tokens.  Kind and page are uniform
+  // over a wave.
   struct Raw {
-    u32x2 k[kPerLane], v[kPerLane];
+    u32x4 u[kUnits];
     float sc;
   };
-  auto fetch = [&](int32_t phys, Raw& r) __attribute__((always_inline)) {
-    const size_t base = (size_t)phys * kv_page_stride + (size_t)kvh * 16 * D;
+  const size_t page_stride = (size_t)KVH * 16 * D;
+  struct Pages {
+    int32_t a, b;
+  };
+  auto page_ids = [&](uint32_t t) __attribute__((always_inline)) {
+    return Pages{sq.pt[min(2 * t, last_page)], sq.pt[min(2 * t + 1, last_page)]};
+  };
+  auto fetch = [&](Pages ph, Raw& r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-      const int u = lane + 64 * i;
-      if (u < kKUnits / kWaves) {
-        const size_t off = base + 8 * (size_t)(wave_unit0 + u);
-        r.k[i] = *(const u32x2*)(sq.k + off);
-        r.v[i] = *(const u32x2*)(sq.v + off);
+    for (int i = 0; i < kUnits; ++i) {
+      const int u0 = i * 64 * W + wave * 64;
+      if (u0 < 4 * D) {
+        const int8_t* base = u0 < 2 * D ? sq.k : sq.v;
+        const int32_t phys = (u0 / D) & 1 ? ph.b : ph.a;
+        r.u[i] = *(const u32x4*)(base + (size_t)phys * page_stride + (size_t)kvh * 16 * D + 16 * (u0 % D + lane));
       }
     }
-    if (wave == 0 && lane < 32) {
+    if (wave == W - 1) {
+      const int32_t phys = lane & 16 ? ph.b : ph.a;
       const size_t si = ((size_t)phys * KVH + kvh) * 16 + (lane & 15);
-      r.sc = lane < 16 ? sq.ks[si] * sm_scale : sq.vs[si];
+      r.sc = hf == 0 ? sq.ks[si] * sm_scale : sq.vs[si];
     }
   };
+  // LDS images: K 16-byte chunk (8 d) q of token t at unit 32 q + (t ^ swz),
+  // V^T chunk (page, half, d) at unit (2 page + half) D + d, where half 0
+  // holds a page's tokens 0..3, 8..11 and half 1 tokens 4..7, 12..15.  The
+  // swizzle keeps the unpacking writes (one token, consecutive chunk pairs)
+  // on distinct banks; the reads are contiguous up to a permutation.
+  constexpr int kRow = D / 16;  // K units per token
+  auto k_swz = [](uint32_t pair) { return D == 64 ? (2 * pair) & 7 : pair & 7; };
   auto stage_in = [&](const Raw& r, int st) __attribute__((always_inline)) {
-    uint8_t* base = lds + st * kStage;
+    uint8_t* kl = lds + st * L::kStage;
+    uint8_t* vl = kl + L::kK;
 #pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-      const int u = lane + 64 * i;
-      if (u < kKUnits / kWaves) {
-        const int g = wave_unit0 + u;
-        // K unit: token g / (D / 8), 8-byte chunk c = kq * kKS + j.
-        const int kt = g / (D / 8), c = g % (D / 8);
-        const u32x2 l = q8x4_to_f16_biased(r.k[i].x), h = q8x4_to_f16_biased(r.k[i].y);
-        const int krow = (c % kKS) * 4 + c / kKS;
-        *(u32x4*)(base + 16 * (krow * 16 + (kt ^ (krow & 15)))) = u32x4{l.x, l.y, h.x, h.y};
-        // V unit: d row g / 2, tokens 8 (g & 1) .. + 7 = kq 2 (g & 1), + 1.
-        const int d = g >> 1, kq0 = 2 * (g & 1);
-        const u32x2 v0 = q8x4_to_bf16_signed(r.v[i].x), v1 = q8x4_to_bf16_signed(r.v[i].y);
-        uint8_t* vb = base + 16 * D * 2;
-        *(u32x2*)(vb + 8 * (((d >> 4) * 4 + kq0) * 16 + ((d & 15) ^ (4 * kq0)))) = v0;
-        *(u32x2*)(vb + 8 * (((d >> 4) * 4 + kq0 + 1) * 16 + ((d & 15) ^ (4 * kq0 + 4)))) = v1;
+    for (int i = 0; i < kUnits; ++i) {
+      const int u0 = i * 64 * W + wave * 64;
+      if (u0 >= 4 * D) continue;
+      const u32x4 w = r.u[i];
+      const int pg = (u0 / D) & 1, u = u0 % D + lane;
+      if (u0 < 2 * D) {
+        const uint32_t t = 16 * pg + u / kRow, pair = u % kRow;
+        uint8_t* dst = kl + 16 * (64 * pair + (t ^ k_swz(pair)));
+        const u32x2 a = q8x4_to_f16_signed(w.x), b = q8x4_to_f16_signed(w.y);
+        const u32x2 c2 = q8x4_to_f16_signed(w.z), d2 = q8x4_to_f16_signed(w.w);
+        *(u32x4*)dst = u32x4{a.x, a.y, b.x, b.y};
+        *(u32x4*)(dst + 512) = u32x4{c2.x, c2.y, d2.x, d2.y};
+      } else {
+        const u32x2 a = q8x4_to_bf16_signed(w.x), b = q8x4_to_bf16_signed(w.y);
+        const u32x2 c2 = q8x4_to_bf16_signed(w.z), d2 = q8x4_to_bf16_signed(w.w);
+        uint8_t* dst = vl + 16 * (2 * pg * D + u);
+        *(u32x4*)dst = u32x4{a.x, a.y, c2.x, c2.y};
+        *(u32x4*)(dst + 16 * D) = u32x4{b.x, b.y, d2.x, d2.y};
       }
     }
-    if (wave == 0 && lane < 32) *(float*)(base + 16 * D * 4 + 4 * lane) = r.sc;
+    if (wave == W - 1) *(float*)(kl + L::kK + L::kV + 4 * lane) = r.sc;
   };
 
-  // Softmax and P'V of page p from LDS stage st.  MASKED is false for pages
-  // every column of the wave sees whole (all but the last few): those skip
-  // the causal compare and select per score.
-  auto compute = [&](uint32_t p, int st, auto masked) __attribute__((always_inline)) {
+  // Softmax and P'V of tile t from LDS stage st.  MASKED is false for tiles
+  // every column of the wave sees whole.
+  auto compute = [&](uint32_t t, int st, auto masked) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked)::value;
-    const uint8_t* base = lds + st * kStage;
+    const uint8_t* base = lds + st * L::kStage;
     const u32x4* kl = (const u32x4*)base;
-    const u32x2* vl = (const u32x2*)(base + 16 * D * 2);
-    const floatx4 kss = *(const floatx4*)(base + 16 * D * 4 + 16 * kq);
-    const floatx4 vs = *(const floatx4*)(base + 16 * D * 4 + 64 + 16 * kq);
-    // S^T[token][col] over D in kKS steps of 32; the blocks' chains are
-    // independent and interleave.
-    floatx4 s4[CB];
+    const u32x4* vl = (const u32x4*)(base + L::kK);
+    const floatx4* sl = (const floatx4*)(base + L::kK + L::kV);
+    // Operands leave LDS ahead of their use, in groups of 8 (the scheduler
+    // would otherwise wait for each one in turn).
+    floatx16 s = floatx16{};
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) s4[cb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < kKS; j0 += kGroup) {
+      u32x4 ka[kGroup];
 #pragma unroll
-    for (int j = 0; j < kKS; ++j) {
-      const u32x4 ka = kl[(j * 4 + kq) * 16 + (tok ^ ((j * 4 + kq) & 15))];
+      for (int j = 0; j < kGroup; ++j) ka[j] = kl[32 * (2 * (j0 + j) + hf) + (lc ^ k_swz(j0 + j))];
+      if constexpr (kAhead > 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) s4[cb] = mfma16x16x32_f16(ka, qb[cb][j], s4[cb]);
+      for (int j = 0; j < kGroup; ++j)
+        s = mfma32x32x16_f16(ka[j], j0 + j < kQReg ? qb[j0 + j < kQReg ? j0 + j : 0] : ql[64 * (j0 + j - kQReg)], s);
     }
-    u32x4 pb[CB];
+    floatx4 ks[4], vs[4];
+    auto load_ks = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      // Columns without a query row hold q = 0: their scores are finite and
-      // their results are never stored.
-      float sc[4];
+      for (int g = 0; g < 4; ++g) ks[g] = sl[2 * g + hf];
+    };
+    auto load_vs = [&](int g0, int g1) __attribute__((always_inline)) {
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        sc[rr] = (s4[cb][rr] - qcorr[cb]) * kss[rr];
-        if constexpr (MASKED) {
-          if (p * 16 + 4 * kq + rr >= visible[cb]) sc[rr] = -INFINITY;
-        }
-      }
-      const float bmax = max4_across_kq(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])));
-      // Lazy rescaling: the reference maximum moves only when a score exceeds
-      // it by more than 2^8, so exp2(s - m) <= 256 stays exact in fp32 and the
-      // pass over every accumulator is rare; the final division by l removes
-      // the choice of reference.  Page 0 holds a visible token for every
-      // column, so m_run is finite from the first page on.
-      const float m_new = bmax > m_run[cb] + 8.0f ? bmax : m_run[cb];
-      const bool moved = m_new != m_run[cb];
-      const float corr = moved ? __builtin_amdgcn_exp2f(m_run[cb] - m_new) : 1.0f;
-      m_run[cb] = m_new;
-      float pw[4];
-      float psum = 0.0f;
+      for (int g = g0; g < g1; ++g) vs[g] = sl[8 + 2 * g + hf];
+    };
+    load_ks();
+    if constexpr (kAhead > 0) load_vs(0, 4);
+    u32x4 va[kDB];
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        // v_exp_f32 directly: arguments are <= 8, exp2(-inf) = 0 for masked
-        // tokens, and a flushed tiny probability is below the fp32
-        // resolution of the running sum.
-        const float e = __builtin_amdgcn_exp2f(sc[rr] - m_new);
-        psum += e;
-        pw[rr] = e * vs[rr];  // fold the V scale
-        if constexpr (MASKED) {
-          if (sc[rr] == -INFINITY) pw[rr] = 0.0f;  // whatever an unwritten slot's scale holds
-        }
-      }
-      l_lane[cb] = l_lane[cb] * corr + psum;
-      if (__builtin_amdgcn_ballot_w64(moved)) {
+    for (int db = 0; db < kAhead; ++db) va[db] = vl[hf * D + 32 * db + lc];
+    if constexpr (kAhead > 0) __builtin_amdgcn_sched_barrier(0);
+    // Element e is token 32 t + 8 (e >> 2) + 4 hf + (e & 3).  Probabilities
+    // against the running reference maximum m_run, which moves only when a
+    // score exceeds it by more than 2^8 (exp2(s - m) <= 256 stays exact in
+    // fp32, and the final division by l removes the choice of reference): a
+    // pass over every accumulator is rare, and without one the column's two
+    // halves need no exchange.  v_exp_f32 directly: exp2(-inf) = 0 for masked
+    // tokens, and a flushed tiny probability is below the fp32 resolution of
+    // the running sum.
+    float p[16];
+    float xmax = -INFINITY;
+    bool ok[16];
 #pragma unroll
-        for (int db = 0; db < kDB; ++db) o[cb][db] *= corr;
-      }
-      // P'^T as bf16 hi + lo (error ~2^-16), both in the K dimension of one
-      // 16x16x32 MFMA: lane (d, kq) supplies A = V^T[d][4 kq .. 4 kq + 3]
-      // twice and B = (hi, lo) of the same four tokens (the legacy 16x16x16
-      // form costs as many cycles as the 16x16x32 one).
-      const uint32_t h01 = pack_bf16x2(pw[0], pw[1]), h23 = pack_bf16x2(pw[2], pw[3]);
-      pb[cb] = u32x4{h01, h23, pack_bf16x2(pw[0] - bf16_lo_f32(h01), pw[1] - bf16_hi_f32(h01)),
-                     pack_bf16x2(pw[2] - bf16_lo_f32(h23), pw[3] - bf16_hi_f32(h23))};
+    for (int e = 0; e < 16; ++e) {
+      float x = __builtin_fmaf(s[e], ks[e >> 2][e & 3], -m_run);
+      ok[e] = !MASKED || 32 * t + 8 * (e >> 2) + 4 * hf + (e & 3) < visible;
+      if (!ok[e]) x = -INFINITY;
+      xmax = fmaxf(xmax, x);
+      if constexpr (kAhead > 0) p[e] = __builtin_amdgcn_exp2f(x);
     }
-    // V unbiased (signed bytes -> bf16, exact): O accumulates only
-    // sum_t v_t p'_t.
+    const bool move = __builtin_amdgcn_ballot_w64(xmax > 8.0f) != 0;
+    if (move) {
+      float bmax = -INFINITY;
 #pragma unroll
-    for (int db = 0; db < kDB; ++db) {
-      const u32x2 va = vl[(db * 4 + kq) * 16 + (tok ^ (4 * kq))];
-      const u32x4 vv = {va.x, va.y, va.x, va.y};
+      for (int e = 0; e < 16; ++e)
+        if (ok[e]) bmax = fmaxf(bmax, s[e] * ks[e >> 2][e & 3]);
+      bmax = max2_across_halves(bmax);
+      const float m_new = bmax > m_run + 8.0f ? bmax : m_run;
+      const float corr = m_new != m_run ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.0f;
+      m_run = m_new;
+      l_lane *= corr;
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) o[cb][db] = mfma16x16x32(vv, pb[cb], o[cb][db]);
+      for (int db = 0; db < kDB; ++db) o[db] *= corr;
     }
+    // D = 256 has no registers for scores beside probabilities, and MFMA
+    // time to spare: it forms the exponents again.
+    if (move || kAhead == 0) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float x = __builtin_fmaf(s[e], ks[e >> 2][e & 3], -m_run);
+        p[e] = __builtin_amdgcn_exp2f(ok[e] ? x : -INFINITY);
+      }
+    }
+    float psum[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      // P' = p * v_scale as bf16 hi + lo (error ~2^-16).
+      uint32_t hi[4], lo[4];
+      if constexpr (kAhead == 0) load_vs(2 * j, 2 * j + 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = 8 * j + 2 * i;
+        psum[0] += p[e];
+        psum[1] += p[e + 1];
+        // A masked token adds nothing, whatever an unwritten slot's scale holds.
+        const float a = ok[e] ? p[e] * vs[e >> 2][e & 3] : 0.0f;
+        const float b = ok[e + 1] ? p[e + 1] * vs[(e + 1) >> 2][(e + 1) & 3] : 0.0f;
+        hi[i] = pack_bf16x2(a, b);
+        // Opaque, or the compiler converts a again on its own to get the low half.
+        asm("" : "+v"(hi[i]));
+        lo[i] = pack_bf16x2(a - bf16_lo_f32(hi[i]), b - bf16_hi_f32(hi[i]));
+      }
+      const u32x4 ph = {hi[0], hi[1], hi[2], hi[3]}, pl = {lo[0], lo[1], lo[2], lo[3]};
+      // V unbiased (signed bytes -> bf16, exact): O accumulates only
+      // sum_t v_t p'_t.
+#pragma unroll
+      for (int db = 0; db < kDB; ++db) {
+        const u32x4 v = j == 0 && db < kAhead ? va[db] : vl[(2 * j + hf) * D + 32 * db + lc];
+        o[db] = mfma32x32x16(v, ph, o[db]);
+        o[db] = mfma32x32x16(v, pl, o[db]);
+      }
+    }
+    l_lane += psum[0] + psum[1];
   };
 
-  // Pipeline, one barrier per page: page p + 1's quarter (fetched a page
-  // earlier) is unpacked into the other stage, page p + 2's quarter is
-  // fetched, then page p is reduced from its stage.  The barrier waits on LDS
-  // only, so the fetch stays in flight across it.
-  Raw raw;
-  if (n_pages > 0) {
-    fetch(sq.pt[0], raw);
+  // Pipeline, one barrier per tile: tile t + 1 (fetched a tile earlier) is
+  // unpacked into the other stage, tile t + 2 is fetched, then tile t is
+  // reduced from its stage.  The barrier waits on LDS only, so the fetch
+  // stays in flight across it.
+  Raw raw{};
+  Pages next{};
+  if (t0 < t1) {
+    fetch(page_ids(t0), raw);
+    if (t0 + 1 < t1) next = page_ids(t0 + 1);
     stage_in(raw, 0);
-    if (n_pages > 1) fetch(sq.pt[1], raw);
+    if (t0 + 1 < t1) fetch(next, raw);
+    if (t0 + 2 < t1) next = page_ids(t0 + 2);
   }
   lds_barrier();
-  int32_t ph_next = n_pages > 2 ? sq.pt[2] : 0;
-  auto step = [&](uint32_t p, auto masked) __attribute__((always_inline)) {
-    const int st = p & 1;
-    if (p + 1 < n_pages) stage_in(raw, st ^ 1);
-    if (p + 2 < n_pages) {
-      fetch(ph_next, raw);
-      if (p + 3 < n_pages) ph_next = sq.pt[p + 3];
+  auto step = [&](uint32_t t, auto masked) __attribute__((always_inline)) {
+    const int st = (t - t0) & 1;
+    if (t + 1 < t1) stage_in(raw, st ^ 1);
+    if (t + 2 < t1) {
+      fetch(next, raw);
+      if (t + 3 < t1) next = page_ids(t + 3);
     }
-    compute(p, st, masked);
+    compute(t, st, masked);
     lds_barrier();
   };
-  // Pages below full_end are visible to every row of the wave.
-  const uint32_t full_end = min(min(args.start + row_base + 1, sq.len) / 16, n_pages);
-  for (uint32_t p = 0; p < full_end; ++p) step(p, BoolTag<false>{});
-  for (uint32_t p = full_end; p < n_pages; ++p) step(p, BoolTag<true>{});
+  // Tiles below full_end are visible to every column of the wave.
+  const uint32_t first_row = min(c0, cols - 1) / gh;
+  const uint32_t full_end = min(max(min(args.start + first_row + 1, sq.len) / 32, t0), t1);
+  for (uint32_t t = t0; t < full_end; ++t) step(t, BoolTag<false>{});
+  for (uint32_t t = full_end; t < t1; ++t) step(t, BoolTag<true>{});
 
-  // O^T lane layout: column col, rows d = 16 db + 4 kq + r.
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) {
-    float l_tot = l_lane[cb] + __shfl_xor(l_lane[cb], 16);
-    l_tot += __shfl_xor(l_tot, 32);
-    if (!col_ok[cb]) continue;
-    const float inv = 1.0f / fmaxf(l_tot, FLT_MIN);
-    const size_t obase = ((size_t)qrow[cb] * H + head) * dr;
+  const float l_tot = l_lane + __shfl_xor(l_lane, 32);
+  if (!col_ok) return;
+  if (S > 1) {
+    // Partials as in decode, row by row: O [row][split][H][D], then (m, l).
+    const size_t pr = ((size_t)row * S + split) * H + head;
+    float* po = args.partials + pr * D;
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t d = 16 * db + 4 * kq + r;
+      for (int g = 0; g < 4; ++g)
+        *(floatx4*)(po + 32 * db + 8 * g + 4 * hf) =
+            floatx4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+    if (hf == 0) *(float2*)(args.partials + (size_t)args.part_rows * H * D + pr * 2) = float2{m_run, l_tot};
+    return;
+  }
+  const float inv = 1.0f / fmaxf(l_tot, FLT_MIN);
+  const size_t obase = ((size_t)row * H + head) * dr;
+  if (args.out8) {  // 8-byte accesses: dr % 8 == 0, o and gate aligned
+    u32x2 gt[kDB][4];
+    if (args.gate) {
+#pragma unroll
+      for (int i = 0; i < kDB * 4; ++i) {
+        const uint32_t d0 = 8 * i + 4 * hf;
+        if (d0 < dr) gt[i >> 2][i & 3] = *(const u32x2*)(args.gate + obase + d0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDB * 4; ++i) {
+      const uint32_t d0 = 8 * i + 4 * hf;
+      if (d0 >= dr) continue;
+      const int db = i >> 2, g = i & 3;
+      const floatx4 v = floatx4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]} * inv;
+      *(u32x2*)(args.o + obase + d0) = args.gate ? gated_bf16x4(v, gt[db][g]) : bf16x4_of(v);
+    }
+  } else {
+#pragma unroll 1
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+      for (int db = 0; db < kDB; ++db) {
+        const uint32_t d = 32 * db + 8 * (e >> 2) + 4 * hf + (e & 3);
         if (d >= dr) continue;
-        float v = o[cb][db][r] * inv;
+        float v = o[db][e] * inv;
         if (args.gate) v *= sigmoid_f(bf16_to_f32(args.gate[obase + d]));
         args.o[obase + d] = f32_to_bf16(v);
       }
   }
 }
 
-template <int D, int CB>
+// The merge for prefills whose splits are few (at most kRowSplits) and rows
+// many: a thread per (row, head, 4 d), every split's load in flight at once.
+// (A workgroup per (row, head, 32 d), as above, is 192000 of them for 1000
+// rows of 24 heads of 256: the dispatch alone took longer than the product.)
+constexpr int kRowSplits = 8;
+template <int D>
+__global__ __launch_bounds__(256) void q8_combine_rows_kernel(AttnArgs args) {
+  const uint32_t H = args.heads, dr = args.head_dim, ns = args.splits;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t pair = i / (D / 4);
+  const uint32_t d0 = 4 * (uint32_t)(i % (D / 4));
+  if (pair >= (size_t)args.rows * H || d0 >= dr) return;
+  const size_t row = pair / H, hh = pair % H;
+  floatx4 ov[kRowSplits];
+  float2 ml[kRowSplits];
+#pragma unroll
+  for (int s = 0; s < kRowSplits; ++s) {
+    if ((uint32_t)s >= ns) break;
+    const size_t pr = (row * ns + s) * H + hh;
+    ov[s] = *(const floatx4*)(args.partials + pr * D + d0);
+    ml[s] = *(const float2*)(args.partials + (size_t)args.part_rows * H * D + pr * 2);
+  }
+  float mx = -FLT_MAX;
+#pragma unroll
+  for (int s = 0; s < kRowSplits; ++s)
+    if ((uint32_t)s < ns) mx = fmaxf(mx, ml[s].x);
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  float L = 0.0f;
+#pragma unroll
+  for (int s = 0; s < kRowSplits; ++s)
+    if ((uint32_t)s < ns) {
+      const float f = exp2f(ml[s].x - mx);
+      acc += ov[s] * f;
+      L += ml[s].y * f;
+    }
+  acc *= 1.0f / fmaxf(L, FLT_MIN);
+  const size_t oi = pair * dr + d0;
+  if (args.out8) {
+    *(u32x2*)(args.o + oi) = args.gate ? gated_bf16x4(acc, *(const u32x2*)(args.gate + oi)) : bf16x4_of(acc);
+  } else {
+    for (int e = 0; e < 4 && d0 + e < dr; ++e) {
+      float v = acc[e];
+      if (args.gate) v *= sigmoid_f(bf16_to_f32(args.gate[oi + e]));
+      args.o[oi + e] = f32_to_bf16(v);
+    }
+  }
+}
+
+template <int D>
+void launch_combine(const AttnArgs& a, uint32_t rows, uint32_t max_split, hipStream_t st) {
+  if (max_split <= 32)
+    hipLaunchKernelGGL(q8_combine_small_kernel<D>, dim3(rows * a.heads * (D / 32)), dim3(64), 0, st, a);
+  else
+    hipLaunchKernelGGL(q8_combine_kernel<D>, dim3(rows * a.heads * (D / 32)), dim3(256), 0, st, a);
+}
+
+template <int D, int W>
 hipError_t launch_prefill(const AttnArgs& a, hipStream_t st) {
-  const uint32_t gh = a.heads / a.kv_heads;
-  const uint32_t rows_per_wg = CB * (16 / gh) * 4;
-  const uint32_t units = a.kv_heads * ((a.rows + rows_per_wg - 1) / rows_per_wg);
-  hipLaunchKernelGGL((q8_prefill_kernel<D, CB>), dim3(units), dim3(256), 0, st, a);
+  const uint32_t cols = a.rows * (a.heads / a.kv_heads);
+  const uint32_t units = a.kv_heads * ((cols + 32 * W - 1) / (32 * W)) * a.splits;
+  hipLaunchKernelGGL((q8_prefill_kernel<D, W>), dim3(units), dim3(64 * W), 0, st, a);
+  if (a.splits > 1 && a.splits <= (uint32_t)kRowSplits) {
+    const size_t items = (size_t)a.rows * a.heads * (D / 4);
+    hipLaunchKernelGGL(q8_combine_rows_kernel<D>, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, a);
+  } else if (a.splits > 1) {
+    launch_combine<D>(a, a.rows, a.splits, st);
+  }
   return hipGetLastError();
 }
 
 template <int D>
 hipError_t launch_attn_d(const AttnArgs& a, uint32_t units, bool need_combine, hipStream_t st) {
   if (a.prefill) {
-    // Column blocks per wave: two up to D = 128 (registers for both blocks'
-    // accumulators), one above; QM38_PREFILL_CB overrides (1, 2, 4).
-    int cb = a.prefill_cb > 0 ? a.prefill_cb : (D <= 128 ? 2 : 1);
-    if (D > 128 && cb > 2) cb = 2;
-    if (cb >= 4 && D <= 128) return launch_prefill<D, (D <= 128 ? 4 : 2)>(a, st);
-    if (cb >= 2) return launch_prefill<D, 2>(a, st);
-    return launch_prefill<D, 1>(a, st);
+    if (a.splits == 0 || (a.splits > 1 && !a.partials)) return hipErrorInvalidValue;
+    return a.wg_waves == 8 ? launch_prefill<D, 8>(a, st) : launch_prefill<D, 4>(a, st);
   }
   if (need_combine && !a.partials) return hipErrorInvalidValue;
   if (a.wg_waves == 8)
@@ -1088,10 +1252,7 @@ hipError_t launch_attn_d(const AttnArgs& a, uint32_t units, bool need_combine, h
   if (need_combine) {
     uint32_t max_split = 0;
     for (uint32_t i = 0; i < a.n_seqs; ++i) max_split = max_split > a.seqs[i].nsplit ? max_split : a.seqs[i].nsplit;
-    if (max_split <= 32)
-      hipLaunchKernelGGL(q8_combine_small_kernel<D>, dim3(a.n_seqs * a.heads * (D / 32)), dim3(64), 0, st, a);
-    else
-      hipLaunchKernelGGL(q8_combine_kernel<D>, dim3(a.n_seqs * a.heads * (D / 32)), dim3(256), 0, st, a);
+    launch_combine<D>(a, a.n_seqs, max_split, st);
   }
   return hipGetLastError();
 }

@@ -293,6 +293,38 @@ qm_status plan_decode_chunk(qm_runtime* rt, qm_kv* const* seqs, uint32_t nb, Dec
   return QM_OK;
 }
 
+// The prefill kernel's launch shape: waves per workgroup (32 columns each; a
+// column is a query head of a row) and the workgroups that share the tiles (32
+// tokens) of a column block.
+//
+// Waves.  Eight share an unpacked tile among 256 columns, four among 128.
+// Head storage of 256 leaves a 4-wave workgroup one wave per SIMD, so it takes
+// eight from 1024 columns on (24 / 4 heads, 300 rows on 4000 tokens: 81 us
+// against 109; 40 rows: 45 against 41).  Narrower heads take eight once those
+// workgroups fill the chip twice (64 / 8 heads of 128, 2048 rows on 4096
+// tokens: 519 against 554 us; 1000 on 1000: 112 against 106).  Heads of 64 keep
+// four (8 heads, 2000 rows on 4000: 68 against 82 us).
+//
+// Splits.  One workgroup per column block fills the chip when the rows are
+// many; otherwise as many as run in one residency round, each with at least
+// four tiles, and none below 16 tiles, where the merge costs more than the
+// walk (512 rows of an empty cache: 37 us in two splits, 35 in one).
+void plan_prefill(const qm_runtime* rt, AttnArgs* at) {
+  const uint32_t D = at->head_dim_pad;
+  const uint64_t tiles = ((uint64_t)at->seqs[0].len + 31) / 32, cus = rt->cu_count;
+  const uint64_t cols = (uint64_t)at->rows * (at->heads / at->kv_heads);
+  auto units = [&](uint32_t waves) { return (cols + 32 * waves - 1) / (32 * waves) * at->kv_heads; };
+  const bool wide = D == 256 ? cols >= 1024 : D == 128 && units(8) >= 2 * cus;
+  at->wg_waves = rt->tune.prefill_waves == 4 || rt->tune.prefill_waves == 8 ? rt->tune.prefill_waves : wide ? 8 : 4;
+  if (rt->tune.prefill_splits > 0) {
+    at->splits = (uint32_t)std::min<uint64_t>(rt->tune.prefill_splits, tiles);
+    return;
+  }
+  const uint64_t u = units(at->wg_waves);
+  const uint64_t room = cus * attn_prefill_waves(D, at->wg_waves) * 4 / at->wg_waves;
+  at->splits = tiles <= 16 || 2 * u > room ? 1 : (uint32_t)std::max<uint64_t>(1, std::min(room / u, tiles / 4));
+}
+
 // Shared validation of qm_attn_decode and its no-allocation twin.
 qm_status check_decode_args(qm_runtime* rt, qm_kv* const* seqs, uint32_t B, const uint16_t* q, const uint16_t* gate,
                             const float* k, const float* v, uint32_t H, const uint16_t* o) {
@@ -642,7 +674,13 @@ qm_status qm_attn_prefill(qm_runtime* rt, qm_kv* seq, const uint16_t* q, const u
   at.rows = M;
   at.start = start;
   at.seqs[0] = sd;
-  at.prefill_cb = rt->tune.prefill_cb;
+  at.out8 = D % 8 == 0 && aligned(o, 8);
+  plan_prefill(rt, &at);
+  if (at.splits > 1) {
+    at.part_rows = M * at.splits;
+    at.partials = (float*)prefill_partials(rt, (size_t)at.part_rows * H * (seq->dp + 2) * sizeof(float));
+    if (!at.partials) at.splits = 1;
+  }
   // A cache owned by another runtime: its pending work comes first.
   if ((st = stream_after(rt, seq->rt)) != QM_OK) return st;
   commit_pages(seq, sd.new_page_first, sd.new_page_count);

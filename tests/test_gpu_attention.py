@@ -308,6 +308,63 @@ def test_prefill_matches_oracle(rt, torch_dev, D, H, KVH, start, M):
     _check_cache(cache, mirror)
 
 
+@pytest.mark.parametrize("D,H,KVH", [(64, 8, 8), (50, 7, 1), (128, 64, 8), (100, 10, 2), (128, 16, 1), (256, 24, 4),
+                                     (204, 15, 3)])
+@pytest.mark.parametrize("waves,splits", [(4, 1), (8, 1), (4, 2), (8, 3), (4, 8), (8, 9), (4, 40)])
+def test_prefill_launch_shapes(rt, torch_dev, D, H, KVH, waves, splits):
+    """Both workgroup widths, unsplit and with every merge (up to 8 splits a
+    thread per output, up to 32 and beyond a wave or workgroup per head slice),
+    splits that see nothing of the early rows, column blocks that cut a row's
+    heads, and outputs without the 8-byte alignment of the vector store."""
+    rng = np.random.default_rng(D + H + waves + splits)
+    start, M = (int(rng.integers(0, 40)), 45) if splits < 8 else (1300, 5)
+    cache = rt.create_q8_kv_state(KVH, D, start + M)
+    mirror = Mirror(KVH, D)
+    _fill(rt, torch_dev, cache, mirror, rng, start, H, KVH, D)
+    with tuned(QM38_PREFILL_WAVES=waves, QM38_PREFILL_SPLITS=splits) as trt:
+        q_bits, q_f, g_bits, g_f, k, v = _rand_qkv(rng, M, H, KVH, D, gate=splits != 3)
+        mirror.append(k, v)
+        ref = mirror.reference(q_f, g_f, start)
+        got = _prefill(trt, torch_dev, cache, q_bits, g_bits, k, v, H)
+        assert_bf16_close(got, ref, what=f"{waves} waves {splits} splits")
+        # The same rows into an output that is only 2-byte aligned: the same bits.
+        cache.truncate(start)
+        flat = empty_bf16((M * H * D + 1,), torch_dev)
+        trt.gqa_attention_q8_prefill(cache, to_dev(q_bits, torch_dev), to_dev(g_bits, torch_dev)
+                                     if g_bits is not None else None, to_dev(k, torch_dev), to_dev(v, torch_dev), H, M,
+                                     flat.data_ptr() + 2)
+        odd = bf16_dev_to_f32(flat[1:]).reshape(M, H, D)
+        assert_bf16_close(odd, ref, what="2-byte aligned output")
+    _check_cache(cache, mirror)
+
+
+def test_prefill_on_two_streams_of_one_runtime(rt, torch_dev):
+    """Split prefills that one runtime enqueues on different streams overlap:
+    each stream has its own partials (five streams: more than are kept)."""
+    D, H, KVH, M, n = 128, 16, 2, 6, 1100
+    rng = np.random.default_rng(17)
+    with tuned() as trt:
+        work = []
+        for i in range(5):
+            cache, mirror = rt.create_q8_kv_state(KVH, D, n + M), Mirror(KVH, D)
+            _fill(rt, torch_dev, cache, mirror, rng, n, H, KVH, D)
+            q_bits, q_f, g_bits, g_f, k, v = _rand_qkv(rng, M, H, KVH, D)
+            mirror.append(k, v)
+            args = [to_dev(a, torch_dev) for a in (q_bits, g_bits, k, v)]
+            work.append((cache, torch.cuda.Stream(), args, empty_bf16((M, H, D), torch_dev),
+                         mirror.reference(q_f, g_f, n)))
+        torch.cuda.synchronize()
+        for _ in range(3):
+            for cache, stream, (q, g, k, v), o, _ref in work:
+                cache.truncate(n)
+                trt.set_stream(stream)
+                trt.gqa_attention_q8_prefill(cache, q, g, k, v, H, M, o)
+        torch.cuda.synchronize()
+        trt.set_stream(torch.cuda.current_stream())
+        for i, (_c, _s, _a, o, ref) in enumerate(work):
+            assert_bf16_close(bf16_dev_to_f32(o), ref, what=f"stream {i}")
+
+
 def test_prefill_equals_decode_steps(rt, torch_dev):
     D, H, KVH, M = 256, 24, 4, 37
     rng = np.random.default_rng(5)
