@@ -60,6 +60,8 @@ struct Tuning {
   int gemm_splits = 0;      // QM38_GEMM_SPLITS: K splits of the prefill GEMM
   int gemm_q = 0;           // QM38_GEMM_Q: stream-K steps per worker
   int gemm_plan_log = 0;    // QM38_GEMM_PLAN_LOG
+  int rows_max = 384;       // QM38_Q4_ROWS_MAX: rows up to which the short-prompt kernel always runs (0: never)
+  int rows_slices = 0;      // QM38_Q4_ROWS_SLICES: K slices of the short-prompt kernel
   int attn_pps = 0;         // QM38_ATTN_PPS: pages per decode split
   int attn_waves = 0;       // QM38_ATTN_WAVES: 4 or 8 waves per decode workgroup
   int attn_target_wgs = 0;  // QM38_ATTN_TARGET_WGS
@@ -112,7 +114,7 @@ void q4_stream_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, 
 // ids[m] from the argmax keys of a kQ4OutArgmax decode launch; zeroes the keys.
 hipError_t launch_q4_argmax_finish(unsigned long long* keys, uint32_t* ids, uint32_t M, hipStream_t stream);
 
-// Prefill Q4 GEMM (M > 16): Y[M][N] = X[M][K] * dequant(W)^T, bf16 out.
+// Prefill Q4 GEMM (M > 16, and not a short prompt): Y[M][N] = X[M][K] * dequant(W)^T, bf16 out.
 // swiglu as above.
 size_t q4_gemm_xh_bytes(uint32_t K, uint32_t M);
 // Split-K partial bytes / counters a GEMM launch needs (0 when it does not split).
@@ -120,6 +122,16 @@ void q4_gemm_workspace(const Q4Job* jobs, int n_jobs, bool swiglu, uint32_t K, u
                        size_t* partial_bytes, size_t* counters);
 hipError_t launch_q4_gemm(const Q4Job* jobs, int n_jobs, bool swiglu, const uint16_t* x,
                           uint32_t K, uint32_t M, const Workspace& ws, hipStream_t stream);
+
+// Q4 projection of a short prompt's rows (q4_rows.hip): 17 rows up to
+// QM38_Q4_ROWS_MAX (more where the weight matrix is small), K a multiple of
+// 256.  Jobs may mix plain projections and gate/up pairs.
+bool q4_rows_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune);
+// K-slice partials and operand-ordered fp16 activations of a launch.
+void q4_rows_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune,
+                       size_t* partial_bytes, size_t* xt_bytes);
+hipError_t launch_q4_rows(const Q4Job* jobs, int n_jobs, const uint16_t* x, uint32_t K, uint32_t M,
+                          const Workspace& ws, hipStream_t stream);
 
 // Residual stream helpers of the decode graph (residual.hip).
 // hidden fp32 [M][n] (+= delta bf16 when delta != NULL), out = bf16 RMSNorm(hidden) * w.

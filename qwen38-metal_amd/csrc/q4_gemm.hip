@@ -1,4 +1,4 @@
-// Q4 prefill projection (M > 16 rows): Y[M][N] = X[M][K] * dequant(W)^T.
+// Q4 prefill projection (more rows than q4_rows.hip takes; any K): Y[M][N] = X[M][K] * dequant(W)^T.
 //
 // Numerics follow the reference's prefill path (qwen38_q4_affine_dequantize_f16
 // + fp16 MPS GEMM, /root/reference/shaders/qwen38.metal:4102-4125,

@@ -112,12 +112,29 @@ qm_status stream_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t
   return hip_check(launch_q4_stream(jobs, n, x, K, M, workspace(rt), rt->stream), what);
 }
 
-// Prefill rows on the GEMM (its split-K workspace and fp16 activation copy
-// first).  swiglu: jobs = {gate, up}; otherwise plain jobs and folded pairs
-// may mix.
+// Prefill rows on the short-prompt kernel or the GEMM (split-K workspace and
+// fp16 activation copy first).  swiglu: jobs = {gate, up}; otherwise plain
+// jobs and folded pairs may mix.
 qm_status gemm_launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, const uint16_t* x, uint32_t K,
                       uint32_t M, const char* what) {
   size_t pbytes = 0, counters = 0;
+  Q4Job pair = jobs[0];
+  if (swiglu) {
+    pair.uw = jobs[1].w;
+    pair.us = jobs[1].s;
+    pair.ub = jobs[1].b;
+    pair.mode = kQ4OutSwiglu;
+  }
+  const Q4Job* folded = swiglu ? &pair : jobs;
+  const int nf = swiglu ? 1 : n;
+  if (q4_rows_supported(folded, nf, K, M, rt->tune)) {
+    size_t xbytes = 0;
+    q4_rows_workspace(folded, nf, K, M, rt->tune, &pbytes, &xbytes);
+    qm_status st = ensure_partials(rt, pbytes);
+    if (st == QM_OK) st = ensure_xh(rt, xbytes);
+    if (st != QM_OK) return st;
+    return hip_check(launch_q4_rows(folded, nf, x, K, M, workspace(rt), rt->stream), what);
+  }
   q4_gemm_workspace(jobs, n, swiglu, K, M, rt->tune, &pbytes, &counters);
   qm_status st = ensure_partials(rt, pbytes);
   if (st == QM_OK) st = ensure_counters(rt, counters);

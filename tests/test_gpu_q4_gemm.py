@@ -254,3 +254,44 @@ def test_mixed_set_in_one_launch(torch_dev, M, knob):
         for o, g, u in ((outs[1], g1, u1), (outs[3], g2, u2)):
             h_ref = oracle.swiglu(oracle.q4_project(xb, *g), oracle.q4_project(xb, *u))
             assert_bf16_close(bf16_dev_to_f32(o), h_ref, what=f"mixed pair M={M} rows {g[0].shape[0]}")
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 65, 96, 97, 200])
+@pytest.mark.parametrize("K,slices", [(256, None), (512, 2), (1280, 1), (2304, 5), (4352, None)])
+def test_short_prompt_kernel(torch_dev, M, K, slices):
+    """17..384 rows with K a multiple of 256 (q4_rows_kernel): one to three row
+    blocks a tile and several row tiles, rows and weight rows that end inside a
+    block, K units (512) cut short, K slices even and uneven, plain jobs and
+    pairs in one launch; within the bar of the oracle and the same bits twice."""
+    import qm38
+    with tuned(QM38_Q4_ROWS_SLICES=slices) as rt:
+        rng = np.random.default_rng(M * 31 + K)
+        ns = (193, 1, 97, 192)
+        mats = [synth.q4_matrix(rng, n, K) for n in ns]
+        up = synth.q4_matrix(rng, 97, K)
+        dev = [_upload(torch_dev, *m) for m in mats + [up]]
+        jobs = [qm38.Runtime.job(*d, n) for d, n in zip(dev, ns + (97,))]
+        xb = synth.bf16_normal(rng, (M, K))
+        xd = to_dev(xb, torch_dev)
+        runs = []
+        for _ in range(2):
+            outs = [empty_bf16((M, n), torch_dev) for n in ns]
+            rt.q4_project_set(jobs[:4], [None, None, jobs[4], None], xd, K, M, outs)
+            runs.append([bf16_dev_to_f32(o) for o in outs])
+        for i, (n, m) in enumerate(zip(ns, mats)):
+            ref = oracle.q4_project(xb, *m)
+            if i == 2:
+                ref = oracle.swiglu(ref, oracle.q4_project(xb, *up))
+            assert_bf16_close(runs[0][i], ref, what=f"M {M} K {K} N {n}")
+            assert np.array_equal(runs[0][i], runs[1][i])
+
+
+@pytest.mark.parametrize("M,N,K", [(384, 64, 512), (385, 64, 512), (500, 300, 1024), (385, 9000, 256)])
+def test_short_prompt_limits(rt, torch_dev, M, N, K):
+    # Either side of the row limit, and more rows of a small matrix (which
+    # stay on the short-prompt kernel) and of one whose tiles need two rounds.
+    rng = np.random.default_rng(M + N)
+    mat = synth.q4_matrix(rng, N, K)
+    xb = synth.bf16_normal(rng, (M, K))
+    (got,) = _project(rt, torch_dev, [mat], xb, M)
+    assert_bf16_close(got, oracle.q4_project(xb, *mat), what=f"M{M} N{N} K{K}")
