@@ -60,6 +60,8 @@ struct Tuning {
   int gemm_splits = 0;      // QM38_GEMM_SPLITS: K splits of the prefill GEMM
   int gemm_q = 0;           // QM38_GEMM_Q: stream-K steps per worker
   int gemm_plan_log = 0;    // QM38_GEMM_PLAN_LOG
+  int lanes_lo = 3;         // QM38_Q4_LANES_LO: fewest activation rows (up to 16) on the LDS-streaming kernel (0: off)
+  int lanes_slices = 0;     // QM38_Q4_LANES_SLICES: its K slices, for matrices of any size
   int rows_max = 384;       // QM38_Q4_ROWS_MAX: rows up to which the short-prompt kernel always runs (0: never)
   int rows_slices = 0;      // QM38_Q4_ROWS_SLICES: K slices of the short-prompt kernel
   int attn_pps = 0;         // QM38_ATTN_PPS: pages per decode split
@@ -122,6 +124,13 @@ void q4_gemm_workspace(const Q4Job* jobs, int n_jobs, bool swiglu, uint32_t K, u
                        size_t* partial_bytes, size_t* counters);
 hipError_t launch_q4_gemm(const Q4Job* jobs, int n_jobs, bool swiglu, const uint16_t* x,
                           uint32_t K, uint32_t M, const Workspace& ws, hipStream_t stream);
+
+// Q4 projection of QM38_Q4_LANES_LO .. 16 rows (q4_lanes.hip) of large matrices,
+// K a multiple of 256, bf16 outputs.  Jobs may mix plain projections and gate/up pairs.
+bool q4_lanes_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune);
+void q4_lanes_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, const Tuning& tune, size_t* partial_bytes);
+hipError_t launch_q4_lanes(const Q4Job* jobs, int n_jobs, const uint16_t* x, uint32_t K, uint32_t M,
+                           const Workspace& ws, hipStream_t stream);
 
 // Q4 projection of a short prompt's rows (q4_rows.hip): 17 rows up to
 // QM38_Q4_ROWS_MAX (more where the weight matrix is small), K a multiple of

@@ -274,6 +274,8 @@ qm::Tuning qm::read_tuning(int cu_count) {
   t.gemm_splits = get("QM38_GEMM_SPLITS", 0);
   t.gemm_q = get("QM38_GEMM_Q", 0);
   t.gemm_plan_log = get("QM38_GEMM_PLAN_LOG", 0);
+  t.lanes_lo = get("QM38_Q4_LANES_LO", t.lanes_lo);
+  t.lanes_slices = get("QM38_Q4_LANES_SLICES", 0);
   t.rows_max = get("QM38_Q4_ROWS_MAX", t.rows_max);
   t.rows_slices = get("QM38_Q4_ROWS_SLICES", 0);
   t.attn_pps = get("QM38_ATTN_PPS", 0);

@@ -154,11 +154,22 @@ qm_status mma_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t* x
   return hip_check(launch_q4_mma(jobs, n, x, K, M, workspace(rt), rt->stream), what);
 }
 
+// Up to 16 rows on the LDS-streaming kernel (its K-slice workspace first).
+qm_status lanes_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t* x, uint32_t K, uint32_t M,
+                       const char* what) {
+  size_t pbytes = 0;
+  q4_lanes_workspace(jobs, n, K, rt->tune, &pbytes);
+  qm_status st = ensure_partials(rt, pbytes);
+  if (st != QM_OK) return st;
+  return hip_check(launch_q4_lanes(jobs, n, x, K, M, workspace(rt), rt->stream), what);
+}
+
 qm_status launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, const uint16_t* x, uint32_t K,
                  uint32_t M, const char* what) {
-  if (M <= 8) {
-    // One or two activation rows: the streaming kernel; up to 8: the MFMA
-    // streaming kernel; both take a gate/up pair as one job.
+  if (M <= kDecodeMaxRows) {
+    // One or two activation rows: the streaming kernel; a few more: the MFMA
+    // streaming kernel; up to 16: the LDS-streaming kernel; all take a gate/up
+    // pair as one job.
     Q4Job sj[kMaxQ4Jobs];
     int ns = 0;
     if (swiglu) {
@@ -171,6 +182,7 @@ qm_status launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, const ui
     } else {
       for (int i = 0; i < n; ++i) sj[ns++] = jobs[i];
     }
+    if (q4_lanes_supported(sj, ns, K, M, rt->tune)) return lanes_launch(rt, sj, ns, x, K, M, what);
     if (M >= 2 && q4_mma_supported(sj, ns, K, M, rt->tune)) return mma_launch(rt, sj, ns, x, K, M, what);
     if (q4_stream_supported(sj, ns, K, M, rt->tune)) return stream_launch(rt, sj, ns, x, K, M, what);
     if (q4_mma_supported(sj, ns, K, M, rt->tune)) return mma_launch(rt, sj, ns, x, K, M, what);
@@ -280,6 +292,8 @@ qm_status qm_q4_project_set(qm_runtime* rt, const qm_q4_job* jobs, const qm_q4_j
     if (ups && ups[i] && (st = check_job_ranges(rt, *ups[i], in_elems, "up")) != QM_OK) return st;
     if ((st = check_range(rt, outputs[i], (uint64_t)M * jobs[i].out_rows * 2, "output")) != QM_OK) return st;
   }
+  if (q4_lanes_supported(q, n_jobs, in_elems, M, rt->tune))
+    return lanes_launch(rt, q, n_jobs, x, in_elems, M, "Q4 set launch");
   if (M >= 2 && q4_mma_supported(q, n_jobs, in_elems, M, rt->tune))
     return mma_launch(rt, q, n_jobs, x, in_elems, M, "Q4 set launch");
   if (q4_stream_supported(q, n_jobs, in_elems, M, rt->tune))

@@ -472,3 +472,49 @@ def test_mma_streaming_rows(torch_dev, M, K, C):
         mrt.q4_project_set([jm, jg], [None, ju], xd, K, M, outs)
         assert np.array_equal(bf16_dev_to_f32(outs[0]), got1[0])
         assert np.array_equal(bf16_dev_to_f32(outs[1]), bf16_dev_to_f32(h))
+
+
+@pytest.mark.parametrize("M", [3, 4, 5, 8, 9, 15, 16])
+@pytest.mark.parametrize("K,slices", [(256, 1), (768, 2), (1280, 1), (2304, 5), (4352, 3)])
+def test_lanes_kernel(torch_dev, M, K, slices):
+    """q4_lanes_kernel (3..16 rows, K a multiple of 256), forced onto small
+    matrices: weight rows that end inside a tile and a block, a pair's boundary
+    inside a wave's rows, K units (512) cut short, scale rows that are only
+    8-byte aligned, slices even and uneven; plain jobs and a pair in one launch,
+    within the bar of the oracle, the same bits twice."""
+    import qm38
+    with tuned(QM38_Q4_LANES_SLICES=slices) as rt:
+        rng = np.random.default_rng(M * 31 + K)
+        ns = (193, 1, 97, 192)
+        mats = [synth.q4_matrix(rng, n, K) for n in ns]
+        up = synth.q4_matrix(rng, 97, K)
+        jobs = [qm38.Runtime.job(*(to_dev(a, torch_dev) for a in m), m[0].shape[0]) for m in mats + [up]]
+        xb = synth.bf16_normal(rng, (M, K))
+        xd = to_dev(xb, torch_dev)
+        runs = []
+        for _ in range(2):
+            outs = [empty_bf16((M, n), torch_dev) for n in ns]
+            rt.q4_project_set(jobs[:4], [None, None, jobs[4], None], xd, K, M, outs)
+            runs.append([bf16_dev_to_f32(o) for o in outs])
+        for i, (n, m) in enumerate(zip(ns, mats)):
+            ref = oracle.q4_project(xb, *m)
+            if i == 2:
+                ref = oracle.swiglu(ref, oracle.q4_project(xb, *up))
+            assert_bf16_close(runs[0][i], ref, what=f"M {M} K {K} N {n}")
+            assert np.array_equal(runs[0][i], runs[1][i])
+
+
+@pytest.mark.parametrize("M", [3, 8, 16])
+def test_large_sets_of_a_few_rows(rt, torch_dev, M):
+    # 128 tiles and more: the route of a layer's set.
+    import qm38
+    rng = np.random.default_rng(M)
+    K, N, I = 512, 13000, 6200
+    mats = [synth.q4_matrix(rng, n, K) for n in (N, I, I)]
+    j, g, u = (qm38.Runtime.job(*(to_dev(a, torch_dev) for a in m), m[0].shape[0]) for m in mats)
+    xb = synth.bf16_normal(rng, (M, K))
+    outs = [empty_bf16((M, N), torch_dev), empty_bf16((M, I), torch_dev)]
+    rt.q4_project_set([j, g], [None, u], to_dev(xb, torch_dev), K, M, outs)
+    y, h = (bf16_dev_to_f32(o) for o in outs)
+    assert_bf16_close(y, oracle.q4_project(xb, *mats[0]), what="plain")
+    assert_bf16_close(h, oracle.swiglu(oracle.q4_project(xb, *mats[1]), oracle.q4_project(xb, *mats[2])), what="pair")
