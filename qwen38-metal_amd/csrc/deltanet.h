@@ -79,5 +79,8 @@ inline size_t dn_chunk_ws_bytes(uint32_t M, uint32_t value_heads) {
 bool dn_step_split(const DnArgs& a);
 
 hipError_t launch_deltanet(const DnArgs& a, hipStream_t st);
+// dst0[0..n0) = src0, dst1[0..n1) = src1 (floats; no overlap) in one launch.
+hipError_t launch_dn_copy(const float* src0, float* dst0, size_t n0, const float* src1, float* dst1, size_t n1,
+                          hipStream_t st);
 
 }  // namespace qm

@@ -1803,6 +1803,27 @@ __global__ __launch_bounds__(kScanThreads) void dn_chunk_scan_kernel(DnArgs a) {
   for (int r = 0; r < 4; ++r) sout[(4 * grp + r) * kCD + col_w + j] = d[r];
 }
 
+// Restores a state image: history and S in one launch (two copies took 4 us
+// and a gap), 16 bytes a thread where the counts and addresses allow.
+struct CopyArgs {
+  const float* src[2];
+  float* dst[2];
+  size_t n[2];  // floats
+};
+__global__ __launch_bounds__(256) void dn_copy_kernel(CopyArgs c) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const bool vec = (((uintptr_t)c.src[k] | (uintptr_t)c.dst[k] | (c.n[k] * 4)) & 15) == 0;
+    const size_t n = vec ? c.n[k] / 4 : c.n[k], step = (size_t)gridDim.x * 256;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
+      if (vec)
+        ((floatx4*)c.dst[k])[i] = ((const floatx4*)c.src[k])[i];
+      else
+        c.dst[k][i] = c.src[k][i];
+    }
+  }
+}
+
 template <int EPT>
 void launch_scan(const DnArgs& a, hipStream_t st) {
   const uint32_t groups = (a.dv + kRowsPerWg - 1) / kRowsPerWg;
@@ -1846,6 +1867,14 @@ void launch_conv_tiled(const DnArgs& a, uint32_t ns, dim3 grid, dim3 block, hipS
     launch_conv_tiled_ns<4>(a, grid, block, st);
 }
 
+hipError_t launch_dn_copy(const float* src0, float* dst0, size_t n0, const float* src1, float* dst1, size_t n1,
+                          hipStream_t st) {
+  const CopyArgs c{{src0, src1}, {dst0, dst1}, {n0, n1}};
+  const size_t blocks = std::min<size_t>((std::max(n0, n1) / 4 + 255) / 256 + 1, 2048);
+  hipLaunchKernelGGL(dn_copy_kernel, dim3((unsigned)blocks), dim3(256), 0, st, c);
+  return hipGetLastError();
+}
+
 hipError_t launch_deltanet(const DnArgs& a, hipStream_t st) {
   if (a.dk == 0 || a.dk > 256 || a.dv == 0 || a.dv > 256 || a.M == 0) return hipErrorInvalidValue;
   // One token with S rows that fit the fused kernel's registers: one launch.
@@ -1869,7 +1898,12 @@ hipError_t launch_deltanet(const DnArgs& a, hipStream_t st) {
   const bool chunked = dn_use_chunked(a);
   if (chunked) {
     // The chunk prep kernel convolves its own inputs.
-  } else if (a.kernel <= kTaps) {
+  } else if (a.kernel <= kTaps && (uint64_t)a.M * units > 24576) {
+    // Many tokens: a wave walks 32 of them with the window in registers and
+    // reads every input once.  Fewer leave the chip to a few waves' chains of
+    // 32 (the whole prefill with 48 units: 5 tokens 16.7 us against 14.3 with a
+    // wave per token, 32 tokens 43.0 against 21.6, 127 70.6 against 53.9, 512
+    // 173 against 172, 800 254 against 262).
     const uint32_t items = ((a.M + kConvTile - 1) / kConvTile) * units;
     const dim3 grid((items + 3) / 4), block(kThreads);
     const uint32_t ns = (std::max(a.dk, a.dv) + 63) / 64;

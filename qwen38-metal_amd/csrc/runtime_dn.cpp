@@ -396,14 +396,9 @@ qm_status qm_dn_snapshot_restore(qm_dn_snapshots* s, uint32_t row, qm_dn_state* 
   }
   DeviceGuard g(s->rt->device);
   if (!g.ok()) return no_device();
-  hipStream_t stream = s->rt->stream;
-  hipError_t e = hipSuccess;
-  if (s->hist_elems)
-    e = hipMemcpyAsync(dst->hist[dst->cur], s->hist + (size_t)row * s->hist_stride, s->hist_elems * sizeof(float),
-                       hipMemcpyDeviceToDevice, stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(dst->rec, s->rec + (size_t)row * s->rec_elems, s->rec_elems * sizeof(float),
-                       hipMemcpyDeviceToDevice, stream);
+  const hipError_t e =
+      launch_dn_copy(s->hist + (size_t)row * s->hist_stride, dst->hist[dst->cur], s->hist_elems,
+                     s->rec + (size_t)row * s->rec_elems, dst->rec, s->rec_elems, s->rt->stream);
   return hip_check(e, "DeltaNet snapshot restore");
 }
 

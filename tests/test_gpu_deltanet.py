@@ -520,3 +520,32 @@ def test_chunked_shadow_prefill_leaves_source(rt, torch_dev):
     ref, _, S_ref = oracle.deltanet_prefill(c, *wts, *[x[9:] for x in acts], 1e-6, hist, S, f64=True)
     _close(got, ref, what="shadow chunked out")
     _close(shadow.read()[1], S_ref, what="shadow chunked state")
+
+
+@pytest.mark.parametrize("ks", [1, 3, 4])
+def test_conv_by_tiles_equals_conv_by_tokens(rt, torch_dev, ks):
+    """A long token-serial prefill convolves 32 tokens a wave, a short one each
+    token by its own wave: one call of 800 rows equals two of 400 bit for bit."""
+    import torch
+    kh, vh, d, M = 12, 24, 64, 800  # 36 units: 28800 > 24576 >= 14400
+    cfg, c = _cfg(kh, vh, d, d, ks)
+    rng = np.random.default_rng(ks)
+    ch = _channels(c)
+    conv = (rng.standard_normal((ch, ks)) * 0.5).astype(np.float32)
+    args = [rng.standard_normal(vh).astype(np.float32) * 0.1, rng.standard_normal(vh).astype(np.float32) * 0.1,
+            np.ones(d, np.float32)]
+    acts = [to_dev(rng.standard_normal(n).astype(np.float32), torch_dev)
+            for n in ((M, ch), (M, vh * d), (M, vh), (M, vh))]
+    with _chunked(False) as trt:
+        w = trt.create_deltanet_weights(cfg, conv, *args)
+        one, two = w.create_state(), w.create_state()
+        out1 = torch.empty((M, vh * d), dtype=torch.float32, device=torch_dev)
+        out2 = torch.empty_like(out1)
+        trt.deltanet_prefill(w, one, *acts, M, 1e-6, out1)
+        for lo in (0, M // 2):
+            trt.deltanet_prefill(w, two, *(x[lo:lo + M // 2].contiguous() for x in acts), M // 2, 1e-6,
+                                 out2[lo:lo + M // 2])
+        torch.cuda.synchronize()
+        assert torch.equal(out1, out2)
+        for x, y in zip(one.read(), two.read()):
+            assert np.array_equal(x, y)
