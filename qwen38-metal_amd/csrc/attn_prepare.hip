@@ -19,7 +19,7 @@
 // Block = (row, head group).  Its threads first build the row's rotation
 // table (one angle, sine and cosine per frequency, shared by all heads) in
 // LDS; then each of the 8 waves prepares every (8 * groups)-th head of the
-// row, issuing the loads of up to 8 heads at once.  Short calls (decode) use
+// row, issuing the loads of up to 6 of its slots at once.  Short calls (decode) use
 // many head groups, long prompts one per row.  A wave holds two heads when
 // head_dim <= 128 (32 lanes each), else one; lane l of a head holds elements
 // 4 l .. 4 l + 3: the sum of squares is a reduction over the head's lanes and
@@ -35,7 +35,7 @@ namespace qm {
 namespace {
 
 constexpr int kPrepWaves = 8;  // waves per block (one block per row)
-constexpr int kPrepBatch = 8;  // heads whose loads a wave issues together
+constexpr int kPrepBatch = 6;  // slots whose loads a wave issues together
 
 __device__ __forceinline__ float pick4(const float (&x)[4], uint32_t k) {
   return k == 0 ? x[0] : k == 1 ? x[1] : k == 2 ? x[2] : x[3];
@@ -68,8 +68,20 @@ __device__ __forceinline__ float half_allsum(float v) {
 // HPW heads per wave: 2 when head_dim <= 128 (32 lanes per head), else 1.
 // For head_dim <= 128 the one-head form's upper 32 lanes add only zeros, so
 // both forms give the same sums bit for bit.
-template <int HPW>
-__global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs a) {
+//
+// ALIGNED: head_dim and half are multiples of 4, so a lane's four elements
+// have their partners in one lane, at the same places (one shuffle each, no
+// choosing), and the lane's sines and cosines are the same for every head and
+// stay in registers.
+//
+// What bounds it: at 2048 rows of 64 / 8 heads of 128 the bytes (147 MB, 29 us
+// at the rate of a large copy) and the arithmetic between them; 36 us, and 47
+// with the general form alone, which shuffles twice per element and reads the
+// table in every head.  At 5 rows of 24 / 4 heads of 256 the chain of loads,
+// angles and shuffles: 4.6 us, and 5.2 with the loads after the angles.  Six
+// slots a batch, or the loads held over sincosf leave room for two blocks a CU.
+template <int HPW, bool ALIGNED>
+__global__ __launch_bounds__(64 * kPrepWaves, ALIGNED ? 6 : 4) void attn_prepare_kernel(PrepArgs a) {
   constexpr uint32_t kLanesPerHead = 64 / HPW;
   __shared__ float cos_s[kPrepMaxHeadDim / 2], sin_s[kPrepMaxHeadDim / 2];
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -78,30 +90,9 @@ __global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs 
   const uint32_t hstride = kPrepWaves * gridDim.y;
   const uint32_t hd = a.head_dim, rd = a.rotary_dim, half = rd / 2;
 
-  // Rotation table of this row: frequency i turns by pos(axis(i)) / theta^(2i/rd).
-  for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
-    uint32_t axis = 0;
-    if (a.has_sections) {
-      if (i % 3 == 1 && i / 3 < a.section1) axis = 1;
-      if (i % 3 == 2 && i / 3 < a.section2) axis = 2;
-    }
-    const uint32_t p = a.positions ? a.positions[(size_t)axis * a.M + row] : a.base + row;
-    // fp64 angle, reduced to [-pi, pi] with a two-part 2 pi (error ~1e-11 rad
-    // at 1e5 rad), then single-precision sine and cosine of the small argument.
-    const double angle = (double)p * a.inv_freq[i];
-    const double turns = rint(angle * 0.15915494309189535);
-    double r = fma(-turns, 6.283185307179586, angle);
-    r = fma(-turns, 2.4492935982947064e-16, r);
-    float sn, cs;
-    sincosf((float)r, &sn, &cs);
-    cos_s[i] = cs;
-    sin_s[i] = sn;
-  }
-  __syncthreads();
-
   const uint32_t units = a.H + a.KVH;  // query heads, then key heads
   const uint32_t slots = (units + HPW - 1) / HPW;  // wave work items of HPW heads
-  const bool vec = hd % 4 == 0;
+  const bool vec = ALIGNED || hd % 4 == 0;
   const uint32_t hl = lane % kLanesPerHead, hsel = lane / kLanesPerHead, base = hsel * kLanesPerHead;
   const uint32_t c0 = 4 * hl;
   const bool mine = c0 < hd;
@@ -112,9 +103,10 @@ __global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs 
     wq[j] = c0 + j < hd ? a.q_norm[c0 + j] : 0.0f;
     wk[j] = c0 + j < hd ? a.k_norm[c0 + j] : 0.0f;
   }
-  for (uint32_t first = blockIdx.y * kPrepWaves + wave; first < slots; first += hstride * kPrepBatch) {
-    // Issue the loads of up to kPrepBatch slots (and the query heads' gates).
-    uint2 in[kPrepBatch], gt[kPrepBatch];
+  // The loads of up to kPrepBatch slots (and the query heads' gates).  The
+  // first batch is in flight while the rotation table is built.
+  uint2 in[kPrepBatch], gt[kPrepBatch];
+  auto issue = [&](uint32_t first) __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < kPrepBatch; ++b) {
       const uint32_t u = (first + hstride * b) * HPW + hsel;
@@ -143,6 +135,46 @@ __global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs 
         }
       }
     }
+  };
+  uint32_t first = blockIdx.y * kPrepWaves + wave;
+  if (first < slots) issue(first);
+
+  // Rotation table of this row: frequency i turns by pos(axis(i)) / theta^(2i/rd).
+  for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
+    uint32_t axis = 0;
+    if (a.has_sections) {
+      if (i % 3 == 1 && i / 3 < a.section1) axis = 1;
+      if (i % 3 == 2 && i / 3 < a.section2) axis = 2;
+    }
+    const uint32_t p = a.positions ? a.positions[(size_t)axis * a.M + row] : a.base + row;
+    // fp64 angle, reduced to [-pi, pi] with a two-part 2 pi (error ~1e-11 rad
+    // at 1e5 rad), then single-precision sine and cosine of the small argument.
+    const double angle = (double)p * a.inv_freq[i];
+    const double turns = rint(angle * 0.15915494309189535);
+    double r = fma(-turns, 6.283185307179586, angle);
+    r = fma(-turns, 2.4492935982947064e-16, r);
+    float sn, cs;
+    sincosf((float)r, &sn, &cs);
+    cos_s[i] = cs;
+    sin_s[i] = sn;
+  }
+  __syncthreads();
+
+  float cs[4], sn[4];  // ALIGNED: this lane's, sn with the sign of its half
+  if constexpr (ALIGNED) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t c = c0 + j, f = c < half ? c : c - half;
+      cs[j] = c < rd ? cos_s[f] : 1.0f;
+      sn[j] = c < rd ? (c < half ? -sin_s[f] : sin_s[f]) : 0.0f;
+    }
+  }
+  const bool rotates = c0 < rd;
+  const int other_lane = (int)(base + (c0 < half ? hl + half / 4 : rotates ? hl - half / 4 : hl));
+  const float inv_hd = 1.0f / (float)hd;
+  const bool pow2 = (hd & (hd - 1)) == 0;  // then the product with 1 / hd is the quotient
+
+  while (first < slots) {
 #pragma unroll
     for (int b = 0; b < kPrepBatch; ++b) {
       const uint32_t slot = first + hstride * b;
@@ -159,13 +191,18 @@ __global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs 
         ss += x[j] * x[j];
       }
       ss = HPW == 2 ? half_allsum(ss) : wave_allsum(ss);
-      const float scale = 1.0f / sqrtf(ss / (float)hd + a.eps);
+      const float scale = 1.0f / sqrtf((pow2 ? ss * inv_hd : ss / (float)hd) + a.eps);
 #pragma unroll
       for (int j = 0; j < 4; ++j) x[j] = mine && c0 + j < hd ? x[j] * scale * (is_q ? wq[j] : wk[j]) : 0.0f;
       float y[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t c = c0 + j;
+        if constexpr (ALIGNED) {
+          const float other = __shfl(x[j], other_lane);  // every lane joins the shuffles
+          y[j] = rotates ? fmaf(other, sn[j], x[j] * cs[j]) : x[j];
+          continue;
+        }
         const float other = partner(x, hl, base, (uint32_t)j, half);  // every lane joins the shuffles
         y[j] = x[j];
         if (c < rd) {
@@ -200,6 +237,8 @@ __global__ __launch_bounds__(64 * kPrepWaves) void attn_prepare_kernel(PrepArgs 
         }
       }
     }
+    first += hstride * kPrepBatch;
+    if (first < slots) issue(first);
   }
 }
 
@@ -221,10 +260,10 @@ hipError_t launch_attn_prepare(const PrepArgs& a, hipStream_t st) {
     const uint32_t max_groups = (slots + kPrepWaves - 1) / kPrepWaves;
     const uint32_t groups = std::max(1u, std::min(max_groups, (1024u + rows - 1) / rows));
     const dim3 grid(rows, groups);
-    if (hpw == 2)
-      hipLaunchKernelGGL(attn_prepare_kernel<2>, grid, dim3(64 * kPrepWaves), 0, st, c);
-    else
-      hipLaunchKernelGGL(attn_prepare_kernel<1>, grid, dim3(64 * kPrepWaves), 0, st, c);
+    const bool aligned = a.head_dim % 4 == 0 && a.rotary_dim % 8 == 0;
+    auto kernel = hpw == 2 ? (aligned ? attn_prepare_kernel<2, true> : attn_prepare_kernel<2, false>)
+                           : (aligned ? attn_prepare_kernel<1, true> : attn_prepare_kernel<1, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kPrepWaves), 0, st, c);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

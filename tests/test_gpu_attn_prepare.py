@@ -81,6 +81,17 @@ def test_matches_oracle(rt, torch_dev, M, H, KVH, hd, rd, mode):
         _check(rt, torch_dev, qg, k, qn, kn, hd, rd, 1e7, sections=(11, 10), positions=pos, what="mrope")
 
 
+@pytest.mark.parametrize("M,H,KVH,hd,rd", [
+    (1100, 128, 8, 64, 64),  # more slots than one batch of loads
+    (9, 7, 1, 128, 128),     # an odd number of heads, two to a wave
+    (4, 3, 1, 100, 24),      # head_dim no power of two
+    (3, 2, 1, 12, 8), (3, 2, 1, 132, 8), (2, 3, 1, 256, 256),
+    (5, 4, 2, 64, 12),       # a partner in another place of its lane
+])
+def test_partner_lanes(rt, torch_dev, M, H, KVH, hd, rd):
+    test_matches_oracle(rt, torch_dev, M, H, KVH, hd, rd, "mrope")
+
+
 def test_prepared_rows_feed_decode_attention(rt, torch_dev):
     # prepare -> qm_attn_decode: the attention output equals the oracle's
     # attention over the oracle-prepared q/k (KV quantised by the same rule).
