@@ -826,7 +826,7 @@ __device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
 // Few rows leave the chip idle if one workgroup walks all tiles (5 rows of
 // 24 / 4 heads on 20001 tokens ran on 4 workgroups, 1570 us), so the tiles
 // are then split over args.splits workgroups, whose (O, m, l) the combine
-// kernel merges (37 us with the merge).
+// kernel merges (33 us with the merge).
 //
 // What bounds it: at 2048 rows on 4096 tokens (64 / 8 heads of 128) about 220
 // VALU operations and 24 MFMAs (768 cycles) per wave and tile, two waves per
@@ -849,7 +849,11 @@ __global__ __launch_bounds__(64 * W, attn_prefill_waves(D, W)) void q8_prefill_k
   constexpr int kDB = D / 32;  // 32-wide d blocks of O^T
   constexpr int kKS = D / 16;  // QK k-steps
   // K operands in registers at a time, and V operands taken ahead of the softmax.
-  constexpr int kGroup = D == 256 ? 1 : kKS < 8 ? kKS : 8, kAhead = D == 256 ? 0 : kDB;
+  // Two waves a SIMD of D = 256 have no registers for either; for one wave, which
+  // has nothing else to cover its LDS reads, they are worth 33 -> 29 us at 5
+  // rows on 20001 tokens (with the waves that have no columns only unpacking).
+  constexpr bool kTight = D == 256 && W == 8;
+  constexpr int kGroup = kTight ? 1 : kKS < 8 ? kKS : 8, kAhead = kTight ? 0 : kDB;
   constexpr int kUnits = (4 * D + 64 * W - 1) / (64 * W);  // 16-byte units of a tile per thread
   __shared__ __attribute__((aligned(16))) uint8_t lds[L::kBytes];
 
@@ -1049,8 +1053,8 @@ __global__ __launch_bounds__(64 * W, attn_prefill_waves(D, W)) void q8_prefill_k
 #pragma unroll
       for (int db = 0; db < kDB; ++db) o[db] *= corr;
     }
-    // D = 256 has no registers for scores beside probabilities, and MFMA
-    // time to spare: it forms the exponents again.
+    // Two waves of D = 256 have no registers for scores beside probabilities,
+    // and MFMA time to spare: they form the exponents again.
     if (move || kAhead == 0) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -1111,7 +1115,11 @@ __global__ __launch_bounds__(64 * W, attn_prefill_waves(D, W)) void q8_prefill_k
       fetch(next, raw);
       if (t + 3 < t1) next = page_ids(t + 3);
     }
-    compute(t, st, masked);
+    // A wave without columns only unpacks (of four, three at 5 rows of 24 / 4
+    // heads).  Not for D = 128: the branch keeps the next tile's loads out of the
+    // product's schedule (300 rows of 64 / 8 heads 65 -> 67 us, 1500 of 16 / 2
+    // 139 -> 168).
+    if (D == 128 || W == 8 || c0 < cols) compute(t, st, masked);
     lds_barrier();
   };
   // Tiles below full_end are visible to every column of the wave.
