@@ -612,7 +612,7 @@ def _counter_rows(d: str, counter: str):
 PROBE_CALLS = 5
 PROBE_FILES = {
     "q4_set": TRAFFIC_FILE,
-    "q4_set_m4": "q4_mma_qkv_gateup_m4_traffic.json",
+    "q4_set_m4": "q4_lanes_qkv_gateup_m4_traffic.json",
     "attn_decode_32k": "q8_decode_attn_32k_traffic.json",
     "attn_prefill_2048": "q8_prefill_attn_2048_on_4k_traffic.json",
     "deltanet_step": "dn_step_traffic.json",
