@@ -86,7 +86,10 @@ typedef struct qm_runtime qm_runtime;
 qm_status qm_runtime_create(int device, qm_runtime** out);
 void qm_runtime_destroy(qm_runtime* rt);
 /* Enqueue all later work of `rt` on `hip_stream` (a hipStream_t; NULL selects
- * the null stream).  The stream must belong to the runtime's device. */
+ * the null stream).  The stream must belong to the runtime's device.  Calls on
+ * different streams overlap, except that a call which uses the runtime's
+ * workspaces (split sums, converted activations, intermediate rows) waits on
+ * the device for what was enqueued on the stream left before it. */
 qm_status qm_runtime_set_stream(qm_runtime* rt, void* hip_stream);
 /* Blocks until all work enqueued by `rt` has finished; surfaces asynchronous
  * kernel failures as QM_ERR_COMMAND_FAILED (the reference checks

@@ -64,7 +64,45 @@ static qm_status capture_guard(qm_runtime* rt, const char* what) {
   return QM_OK;
 }
 
+qm_status qm::order_workspaces(qm_runtime* rt) {
+  if (rt->ws_used && !rt->ws_wait && !rt->ws_sync) return QM_OK;
+  // A captured use runs when its graph does; the caller orders that.
+  if (rt->device < 0 || stream_capturing(rt->stream)) return QM_OK;
+  if (rt->ws_sync) {
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) return hip_check(e, "workspace order");
+    rt->ws_sync = rt->ws_wait = false;
+  }
+  if (rt->ws_wait) {
+    const hipError_t e = hipStreamWaitEvent(rt->stream, rt->ws_event, 0);
+    if (e != hipSuccess) return hip_check(e, "workspace order");
+    rt->ws_wait = false;
+  }
+  rt->ws_used = true;
+  return QM_OK;
+}
+
+// The current stream is about to be left: later uses come after its own.
+static void leave_stream(qm_runtime* rt) {
+  if (!rt->ws_used) return;
+  rt->ws_used = false;
+  qm::DeviceGuard g(rt->device);
+  // Nothing can be recorded on a stream under capture, nor on one that no
+  // longer exists.
+  bool recorded = false;
+  if (g.ok() && !qm::stream_capturing(rt->stream)) {
+    hipError_t e = hipSuccess;
+    if (!rt->ws_event) e = hipEventCreateWithFlags(&rt->ws_event, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(rt->ws_event, rt->stream);
+    recorded = e == hipSuccess;
+    if (!recorded) (void)hipGetLastError();
+  }
+  (recorded ? rt->ws_wait : rt->ws_sync) = true;
+}
+
 qm_status qm::ensure_scratch(qm_runtime* rt, size_t bytes) {
+  if (bytes)
+    if (qm_status st_ord = order_workspaces(rt); st_ord != QM_OK) return st_ord;
   if (rt->scratch_bytes >= bytes) return QM_OK;
   if (rt->device < 0) return no_device();
   if (qm_status st_cap = capture_guard(rt, "ensure_scratch"); st_cap != QM_OK) return st_cap;
@@ -85,6 +123,8 @@ qm_status qm::ensure_scratch(qm_runtime* rt, size_t bytes) {
 }
 
 qm_status qm::ensure_partials(qm_runtime* rt, size_t bytes) {
+  if (bytes)
+    if (qm_status st_ord = order_workspaces(rt); st_ord != QM_OK) return st_ord;
   if (rt->partial_bytes >= bytes) return QM_OK;
   if (rt->device < 0) return no_device();
   if (qm_status st_cap = capture_guard(rt, "ensure_partials"); st_cap != QM_OK) return st_cap;
@@ -104,6 +144,8 @@ qm_status qm::ensure_partials(qm_runtime* rt, size_t bytes) {
 }
 
 qm_status qm::ensure_xh(qm_runtime* rt, size_t bytes) {
+  if (bytes)
+    if (qm_status st_ord = order_workspaces(rt); st_ord != QM_OK) return st_ord;
   if (rt->xh_bytes >= bytes) return QM_OK;
   if (rt->device < 0) return no_device();
   if (qm_status st_cap = capture_guard(rt, "ensure_xh"); st_cap != QM_OK) return st_cap;
@@ -122,6 +164,8 @@ qm_status qm::ensure_xh(qm_runtime* rt, size_t bytes) {
 }
 
 qm_status qm::ensure_counters(qm_runtime* rt, size_t count) {
+  if (count)
+    if (qm_status st_ord = order_workspaces(rt); st_ord != QM_OK) return st_ord;
   if (rt->counter_count >= count) return QM_OK;
   if (rt->device < 0) return no_device();
   if (qm_status st_cap = capture_guard(rt, "ensure_counters"); st_cap != QM_OK) return st_cap;
@@ -208,6 +252,7 @@ qm_status qm::stream_after(qm_runtime* waiter, qm_runtime* signaler) {
 }
 
 qm_status qm::ensure_keys(qm_runtime* rt) {
+  if (qm_status st_ord = order_workspaces(rt); st_ord != QM_OK) return st_ord;
   if (rt->keys) return QM_OK;
   if (rt->device < 0) return no_device();
   if (qm_status st_cap = capture_guard(rt, "ensure_keys"); st_cap != QM_OK) return st_cap;
@@ -357,13 +402,18 @@ void qm_runtime_destroy(qm_runtime* rt) {
   }
   DeviceGuard g(rt->device);
   (void)hipStreamSynchronize(rt->stream);
+  if (rt->ws_wait) (void)hipEventSynchronize(rt->ws_event);
+  if (rt->ws_sync) (void)hipDeviceSynchronize();
   qm::release_buffers(rt);
+  if (rt->ws_event) (void)hipEventDestroy(rt->ws_event);
   if (rt->order_event) (void)hipEventDestroy(rt->order_event);
   delete rt;
 }
 
 qm_status qm_runtime_set_stream(qm_runtime* rt, void* hip_stream) {
   if (!rt) return fail(QM_ERR_NULL_POINTER, "runtime is NULL");
+  if (rt->stream == (hipStream_t)hip_stream) return QM_OK;
+  leave_stream(rt);
   rt->stream = (hipStream_t)hip_stream;
   return QM_OK;
 }

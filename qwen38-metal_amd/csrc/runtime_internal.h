@@ -12,17 +12,23 @@ struct qm_runtime {
   int cu_count = 256;
   qm::Tuning tune{};  // planner overrides, read once at creation
   hipStream_t stream = nullptr;
+  // The workspaces below (scratch .. xh, and keys) are one of each per runtime:
+  // calls on one stream use them in turn, and after qm_runtime_set_stream the
+  // first use waits for the uses on the stream that was left (order_workspaces).
+  bool ws_used = false;            // used on `stream` since it was set
+  bool ws_wait = false;            // the next use comes after ws_event
+  bool ws_sync = false;            // the next use comes after all the device's work
+  hipEvent_t ws_event = nullptr;   // the last use on the streams left so far
   // Grow-only scratch used by calls that need an intermediate buffer (the
-  // MLP's h, attention split partials).  Calls on one runtime are serialised
-  // on its stream, so one buffer suffices.
+  // MLP's h, the DeltaNet conv output).
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
   // Zero-initialised completion counters for kernels whose last workgroup
   // combines partial results; every such kernel leaves them at zero again.
   unsigned int* counters = nullptr;
   size_t counter_count = 0;
-  // Split-K partial results of the kernels that combine them in their last
-  // workgroup (no zeroing needed: every slot is written before it is read).
+  // Partial results of kernels that split a sum over workgroups (no zeroing
+  // needed: every slot is written before it is read).
   void* partials = nullptr;
   size_t partial_bytes = 0;
   // fp16 activations of the prefill GEMM (separate from `scratch`, which may
@@ -53,6 +59,10 @@ qm_status fail(qm_status status, const char* fmt, ...);
 qm_status hip_check(hipError_t err, const char* what);
 // QM_ERR_NO_DEVICE for a call on a runtime created without a device.
 qm_status no_device();
+// Puts the workspace use that the caller is about to enqueue behind the uses on
+// streams the runtime has left.  The ensure_ functions call it, so every use
+// begins with one of them.
+qm_status order_workspaces(qm_runtime* rt);
 qm_status ensure_scratch(qm_runtime* rt, size_t bytes);
 qm_status ensure_partials(qm_runtime* rt, size_t bytes);
 qm_status ensure_counters(qm_runtime* rt, size_t count);
