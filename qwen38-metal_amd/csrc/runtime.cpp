@@ -9,7 +9,6 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <algorithm>
 #include <string>
 
 using namespace qm;
@@ -187,44 +186,9 @@ qm_status qm::ensure_counters(qm_runtime* rt, size_t count) {
   return QM_OK;
 }
 
-void* qm::prefill_partials(qm_runtime* rt, size_t bytes) {
-  // A per-thread default stream is several streams under one handle.
-  if (rt->device < 0 || rt->stream == hipStreamPerThread || stream_capturing(rt->stream)) return nullptr;
-  auto& spaces = rt->prefill_spaces;
-  qm_runtime::PrefillSpace* own = nullptr;
-  for (auto& p : spaces)
-    if (p.stream == rt->stream) own = &p;
-  if (own && own->bytes >= bytes) return own->ptr;
-  if (!own) {
-    if (spaces.size() >= qm_runtime::kMaxPrefillSpaces) {
-      if (hipDeviceSynchronize() != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-      }
-      for (auto& p : spaces) (void)hipFree(p.ptr);
-      spaces.clear();
-    }
-    spaces.push_back({rt->stream, nullptr, 0});
-    own = &spaces.back();
-  }
-  if (own->ptr) {
-    // Work already enqueued may still use the old buffer.
-    if (hipStreamSynchronize(rt->stream) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    (void)hipFree(own->ptr);
-    own->ptr = nullptr;
-    own->bytes = 0;
-  }
-  const size_t want = (std::max<size_t>(bytes, 4u << 20) + 255) & ~size_t(255);
-  if (hipMalloc(&own->ptr, want) != hipSuccess) {
-    (void)hipGetLastError();
-    own->ptr = nullptr;
-    return nullptr;
-  }
-  own->bytes = want;
-  return own->ptr;
+bool qm::try_partials(qm_runtime* rt, size_t bytes) {
+  if (rt->device < 0 || rt->stream == hipStreamPerThread || stream_capturing(rt->stream)) return false;
+  return ensure_partials(rt, bytes) == QM_OK;
 }
 
 bool qm::stream_capturing(hipStream_t s) {
@@ -274,9 +238,6 @@ void qm::release_buffers(qm_runtime* rt) {
   if (rt->partials) (void)hipFree(rt->partials);
   if (rt->xh) (void)hipFree(rt->xh);
   if (rt->keys) (void)hipFree(rt->keys);
-  if (rt->prefill_spaces.size() > 1) (void)hipDeviceSynchronize();  // other streams' prefills
-  for (auto& p : rt->prefill_spaces) (void)hipFree(p.ptr);
-  rt->prefill_spaces.clear();
   rt->keys = nullptr;
   rt->scratch = rt->counters = nullptr;
   rt->partials = rt->xh = nullptr;

@@ -2,8 +2,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <vector>
-
 #include "../../include/qm38.h"
 #include "internal.h"
 
@@ -35,17 +33,6 @@ struct qm_runtime {
   // hold the MLP's h while h itself is converted).
   void* xh = nullptr;
   size_t xh_bytes = 0;
-  // Split partials of attention prefills, one buffer per stream the runtime
-  // was used on: prefills enqueued on different streams (set_stream between
-  // them) overlap, so they cannot share one.  At most kMaxPrefillSpaces; a
-  // further stream waits for the device and starts over.
-  struct PrefillSpace {
-    hipStream_t stream;
-    void* ptr;
-    size_t bytes;
-  };
-  static constexpr size_t kMaxPrefillSpaces = 4;
-  std::vector<PrefillSpace> prefill_spaces;
   // Argmax keys of qm_q4_argmax (one uint64 per row of a 16-row chunk); zero
   // between calls, like the counters.
   unsigned long long* keys = nullptr;
@@ -68,10 +55,11 @@ qm_status ensure_partials(qm_runtime* rt, size_t bytes);
 qm_status ensure_counters(qm_runtime* rt, size_t count);
 qm_status ensure_xh(qm_runtime* rt, size_t bytes);
 qm_status ensure_keys(qm_runtime* rt);
-// The runtime's prefill partials for its current stream, at least `bytes`; NULL
-// where they cannot be had (out of memory, a capturing or per-thread stream):
-// the prefill then runs unsplit.
-void* prefill_partials(qm_runtime* rt, size_t bytes);
+// ensure_partials for callers that have another way: false where the partials
+// cannot be had.  Also false where a call's two launches could not keep them to
+// themselves: on a per-thread default stream, one handle for several streams,
+// and under capture, where the graph would keep a pointer that growth frees.
+bool try_partials(qm_runtime* rt, size_t bytes);
 // Workspace handed to kernels that split work across workgroups.
 Workspace workspace(qm_runtime* rt);
 // The device-allocation range checks of every Q4 entry point for one job of

@@ -325,6 +325,15 @@ void plan_prefill(const qm_runtime* rt, AttnArgs* at) {
   at->splits = tiles <= 16 || 2 * u > room ? 1 : (uint32_t)std::max<uint64_t>(1, std::min(room / u, tiles / 4));
 }
 
+// Partials of any split prefill with this head storage: its workgroups fit one
+// residency round, so their columns are bounded whatever the rows and the
+// cache's length.  Sized to that at first use (34 MB with heads of 128, 68 with
+// 256), the buffer does not grow with the cache: growth waits for the stream.
+size_t prefill_partial_bytes(const qm_runtime* rt, uint32_t D) {
+  const size_t waves = 4 * (size_t)std::max(attn_prefill_waves(D, 4), attn_prefill_waves(D, 8)) * rt->cu_count;
+  return waves * 32 * (D + 2) * sizeof(float);
+}
+
 // Shared validation of qm_attn_decode and its no-allocation twin.
 qm_status check_decode_args(qm_runtime* rt, qm_kv* const* seqs, uint32_t B, const uint16_t* q, const uint16_t* gate,
                             const float* k, const float* v, uint32_t H, const uint16_t* o) {
@@ -678,8 +687,11 @@ qm_status qm_attn_prefill(qm_runtime* rt, qm_kv* seq, const uint16_t* q, const u
   plan_prefill(rt, &at);
   if (at.splits > 1) {
     at.part_rows = M * at.splits;
-    at.partials = (float*)prefill_partials(rt, (size_t)at.part_rows * H * (seq->dp + 2) * sizeof(float));
-    if (!at.partials) at.splits = 1;
+    const size_t bytes = (size_t)at.part_rows * H * (seq->dp + 2) * sizeof(float);
+    if (try_partials(rt, std::max(bytes, prefill_partial_bytes(rt, seq->dp))) || try_partials(rt, bytes))
+      at.partials = (float*)rt->partials;
+    else
+      at.splits = 1;
   }
   // A cache owned by another runtime: its pending work comes first.
   if ((st = stream_after(rt, seq->rt)) != QM_OK) return st;

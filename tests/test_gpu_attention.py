@@ -339,8 +339,8 @@ def test_prefill_launch_shapes(rt, torch_dev, D, H, KVH, waves, splits):
 
 
 def test_prefill_on_two_streams_of_one_runtime(rt, torch_dev):
-    """Split prefills that one runtime enqueues on different streams overlap:
-    each stream has its own partials (five streams: more than are kept)."""
+    """Split prefills that one runtime enqueues on five streams in turn: one set
+    of partials, in stream order."""
     D, H, KVH, M, n = 128, 16, 2, 6, 1100
     rng = np.random.default_rng(17)
     with tuned() as trt:

@@ -59,3 +59,29 @@ def test_workspaces_on_streams_in_turn(torch_dev, M, N, K, env):
         for ref, o in zip(alone, outs):
             for y in o:
                 assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("D,H,KVH,M", [(256, 24, 4, 5), (128, 16, 2, 8), (64, 8, 8, 40), (256, 24, 4, 300)])
+def test_prefill_partials_are_sized_once(torch_dev, D, H, KVH, M):
+    """A split prefill's partials do not grow with the cache (growing waits for
+    the stream), nor with the streams that the runtime is used on."""
+    import torch
+    rng = np.random.default_rng(D + M)
+    with tuned() as rt:
+        cache = rt.create_q8_kv_state(KVH, D, 9000)
+        cache.reserve(9000)
+        f32 = [to_dev(rng.standard_normal((4200, KVH, D)).astype(np.float32), torch_dev) for _ in range(2)]
+        q = to_dev(synth.bf16_normal(rng, (4200, H, D)), torch_dev)
+        o = empty_bf16((4200, H, D), torch_dev)
+        rt.gqa_attention_q8_prefill(cache, q, None, *f32, H, 1100, o)
+        streams = [torch.cuda.Stream() for _ in range(5)]
+        free = []
+        for i in range(20):
+            rt.set_stream(streams[i % 5])
+            rt.gqa_attention_q8_prefill(cache, q, None, *f32, H, M, o)
+            torch.cuda.synchronize()
+            free.append(torch.cuda.mem_get_info()[0])
+            rt.gqa_attention_q8_prefill(cache, q, None, *f32, H, 90, o)  # a longer cache
+        torch.cuda.synchronize()
+        rt.set_stream(torch.cuda.current_stream())
+        assert len(set(free[5:])) == 1  # a stream's first launch takes memory of its own
