@@ -112,9 +112,10 @@ qm_status stream_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t
   return hip_check(launch_q4_stream(jobs, n, x, K, M, workspace(rt), rt->stream), what);
 }
 
-// Prefill rows on the short-prompt kernel or the GEMM (split-K workspace and
-// fp16 activation copy first).  swiglu: jobs = {gate, up}; otherwise plain
-// jobs and folded pairs may mix.
+// Prefill rows on the short-prompt kernel, or the GEMM where that one does not
+// apply or its workspace cannot be had (split-K workspace and fp16 activation
+// copy first).  swiglu: jobs = {gate, up}; otherwise plain jobs and folded
+// pairs may mix.
 qm_status gemm_launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, const uint16_t* x, uint32_t K,
                       uint32_t M, const char* what) {
   size_t pbytes = 0, counters = 0;
@@ -132,8 +133,7 @@ qm_status gemm_launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, con
     q4_rows_workspace(folded, nf, K, M, rt->tune, &pbytes, &xbytes);
     qm_status st = ensure_partials(rt, pbytes);
     if (st == QM_OK) st = ensure_xh(rt, xbytes);
-    if (st != QM_OK) return st;
-    return hip_check(launch_q4_rows(folded, nf, x, K, M, workspace(rt), rt->stream), what);
+    if (st == QM_OK) return hip_check(launch_q4_rows(folded, nf, x, K, M, workspace(rt), rt->stream), what);
   }
   q4_gemm_workspace(jobs, n, swiglu, K, M, rt->tune, &pbytes, &counters);
   qm_status st = ensure_partials(rt, pbytes);
@@ -154,13 +154,17 @@ qm_status mma_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t* x
   return hip_check(launch_q4_mma(jobs, n, x, K, M, workspace(rt), rt->stream), what);
 }
 
-// Up to 16 rows on the LDS-streaming kernel (its K-slice workspace first).
+// Up to 16 rows on the LDS-streaming kernel, unless its K slices have no
+// workspace (graph capture, out of memory): the other kernels of these rows
+// then take the call.  *done: launched, or failed to.
 qm_status lanes_launch(qm_runtime* rt, const Q4Job* jobs, int n, const uint16_t* x, uint32_t K, uint32_t M,
-                       const char* what) {
+                       const char* what, bool* done) {
+  *done = false;
+  if (!q4_lanes_supported(jobs, n, K, M, rt->tune)) return QM_OK;
   size_t pbytes = 0;
   q4_lanes_workspace(jobs, n, K, rt->tune, &pbytes);
-  qm_status st = ensure_partials(rt, pbytes);
-  if (st != QM_OK) return st;
+  if (pbytes && !try_partials(rt, pbytes)) return QM_OK;
+  *done = true;
   return hip_check(launch_q4_lanes(jobs, n, x, K, M, workspace(rt), rt->stream), what);
 }
 
@@ -182,7 +186,9 @@ qm_status launch(qm_runtime* rt, const Q4Job* jobs, int n, bool swiglu, const ui
     } else {
       for (int i = 0; i < n; ++i) sj[ns++] = jobs[i];
     }
-    if (q4_lanes_supported(sj, ns, K, M, rt->tune)) return lanes_launch(rt, sj, ns, x, K, M, what);
+    bool done;
+    const qm_status st = lanes_launch(rt, sj, ns, x, K, M, what, &done);
+    if (done) return st;
     if (M >= 2 && q4_mma_supported(sj, ns, K, M, rt->tune)) return mma_launch(rt, sj, ns, x, K, M, what);
     if (q4_stream_supported(sj, ns, K, M, rt->tune)) return stream_launch(rt, sj, ns, x, K, M, what);
     if (q4_mma_supported(sj, ns, K, M, rt->tune)) return mma_launch(rt, sj, ns, x, K, M, what);
@@ -292,8 +298,9 @@ qm_status qm_q4_project_set(qm_runtime* rt, const qm_q4_job* jobs, const qm_q4_j
     if (ups && ups[i] && (st = check_job_ranges(rt, *ups[i], in_elems, "up")) != QM_OK) return st;
     if ((st = check_range(rt, outputs[i], (uint64_t)M * jobs[i].out_rows * 2, "output")) != QM_OK) return st;
   }
-  if (q4_lanes_supported(q, n_jobs, in_elems, M, rt->tune))
-    return lanes_launch(rt, q, n_jobs, x, in_elems, M, "Q4 set launch");
+  bool done;
+  st = lanes_launch(rt, q, n_jobs, x, in_elems, M, "Q4 set launch", &done);
+  if (done) return st;
   if (M >= 2 && q4_mma_supported(q, n_jobs, in_elems, M, rt->tune))
     return mma_launch(rt, q, n_jobs, x, in_elems, M, "Q4 set launch");
   if (q4_stream_supported(q, n_jobs, in_elems, M, rt->tune))

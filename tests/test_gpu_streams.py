@@ -85,3 +85,42 @@ def test_prefill_partials_are_sized_once(torch_dev, D, H, KVH, M):
         torch.cuda.synchronize()
         rt.set_stream(torch.cuda.current_stream())
         assert len(set(free[5:])) == 1  # a stream's first launch takes memory of its own
+
+
+@pytest.mark.parametrize("M,specs,K", [
+    (12, [(10000, False)], 1536),              # medium matrices
+    (9, [(3200, False)], 9216),                # long K
+    (16, [(3000, False), (4000, True)], 1536), # a set
+])
+def test_few_rows_capture_without_a_warm_call(torch_dev, M, specs, K):
+    """A fresh runtime's first projection of a few rows may be a captured one:
+    where the kernel's K slices have no workspace another kernel takes the call.
+    Replayed with eager work in between."""
+    import torch
+    rng = np.random.default_rng(M)
+    with tuned() as rt, tuned() as eager:
+        mats = [synth.q4_matrix(rng, n, K) for n, _ in specs]
+        ups = [synth.q4_matrix(rng, n, K) if pair else None for n, pair in specs]
+        jobs, upj = [_job(m, torch_dev) for m in mats], [_job(u, torch_dev) if u else None for u in ups]
+        x = to_dev(synth.bf16_normal(rng, (M, K)), torch_dev)
+        outs = [empty_bf16((M, n), torch_dev) for n, _ in specs]
+        refs = [empty_bf16((M, n), torch_dev) for n, _ in specs]
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            rt.set_stream(torch.cuda.current_stream())
+            rt.q4_project_set(jobs, upj, x, K, M, outs)
+        rt.set_stream(torch.cuda.current_stream())
+        for i in range(3):
+            xb = synth.bf16_normal(rng, (M, K))
+            x.copy_(to_dev(xb, torch_dev))
+            eager.q4_project_set(jobs, upj, x, K, M, refs)
+            graph.replay()
+            torch.cuda.synchronize()
+            for o, r, m, u in zip(outs, refs, mats, ups):
+                ref = oracle.q4_project(xb, *m)
+                if u is not None:
+                    ref = oracle.swiglu(ref, oracle.q4_project(xb, *u))
+                assert_bf16_close(bf16_dev_to_f32(o), ref, what=f"replay {i}")
+                assert_bf16_close(bf16_dev_to_f32(r), ref, what=f"eager {i}")
+                o.fill_(-1)
