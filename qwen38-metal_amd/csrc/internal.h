@@ -62,8 +62,8 @@ struct Tuning {
   int gemm_plan_log = 0;    // QM38_GEMM_PLAN_LOG
   int lanes_lo = 3;         // QM38_Q4_LANES_LO: fewest activation rows (up to 16) on the LDS-streaming kernel (0: off)
   int lanes_slices = 0;     // QM38_Q4_LANES_SLICES: its K slices, for matrices of any size
-  int rows_max = 384;       // QM38_Q4_ROWS_MAX: rows up to which the short-prompt kernel always runs (0: never)
-  int rows_slices = 0;      // QM38_Q4_ROWS_SLICES: K slices of the short-prompt kernel
+  int rows_max = 384;       // QM38_Q4_ROWS_MAX: rows up to which the short-prompt kernel competes with the GEMM (0: never)
+  int rows_slices = 0;      // QM38_Q4_ROWS_SLICES: its K slices, for any call of up to that many rows
   int attn_pps = 0;         // QM38_ATTN_PPS: pages per decode split
   int attn_waves = 0;       // QM38_ATTN_WAVES: 4 or 8 waves per decode workgroup
   int attn_target_wgs = 0;  // QM38_ATTN_TARGET_WGS
@@ -116,12 +116,20 @@ void q4_stream_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, 
 // ids[m] from the argmax keys of a kQ4OutArgmax decode launch; zeroes the keys.
 hipError_t launch_q4_argmax_finish(unsigned long long* keys, uint32_t* ids, uint32_t M, hipStream_t stream);
 
-// Prefill Q4 GEMM (M > 16, and not a short prompt): Y[M][N] = X[M][K] * dequant(W)^T, bf16 out.
+// Prefill Q4 GEMM (M > 16, where q4_rows_supported is false): Y[M][N] = X[M][K] * dequant(W)^T, bf16 out.
 // swiglu as above.
 size_t q4_gemm_xh_bytes(uint32_t K, uint32_t M);
 // Split-K partial bytes / counters a GEMM launch needs (0 when it does not split).
 void q4_gemm_workspace(const Q4Job* jobs, int n_jobs, bool swiglu, uint32_t K, uint32_t M, const Tuning& tune,
                        size_t* partial_bytes, size_t* counters);
+// A launch's estimated time; pairs as one job each (kQ4OutSwiglu).
+double q4_gemm_us(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune);
+// How full a round of `wgs` workgroups leaves the chip, for those estimates: 0
+// up to five eighths of the CUs, 1 with all of them.
+inline double wave_fill(double wgs, double cus) {
+  const double f = (wgs / cus - 0.625) / 0.375;
+  return f > 0.0 ? f : 0.0;
+}
 hipError_t launch_q4_gemm(const Q4Job* jobs, int n_jobs, bool swiglu, const uint16_t* x,
                           uint32_t K, uint32_t M, const Workspace& ws, hipStream_t stream);
 
@@ -133,8 +141,9 @@ hipError_t launch_q4_lanes(const Q4Job* jobs, int n_jobs, const uint16_t* x, uin
                            const Workspace& ws, hipStream_t stream);
 
 // Q4 projection of a short prompt's rows (q4_rows.hip): 17 rows up to
-// QM38_Q4_ROWS_MAX (more where the weight matrix is small), K a multiple of
-// 256.  Jobs may mix plain projections and gate/up pairs.
+// QM38_Q4_ROWS_MAX where the GEMM is not the faster (more where the weight
+// matrix is small), K a multiple of 256.  Jobs may mix plain projections and
+// gate/up pairs (one job each).
 bool q4_rows_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune);
 // K-slice partials and operand-ordered fp16 activations of a launch.
 void q4_rows_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune,

@@ -1,4 +1,5 @@
-// Q4 projection of a short prompt's rows (17 .. 128, or a few times that):
+// Q4 projection of a short prompt's rows (17 .. 128, or a few times that where
+// the tiles suit the chip; q4_rows_supported has the line):
 // Y[M][N] = X[M][K] * dequant(W)^T with the GEMM's numerics (q4_gemm.hip):
 // weights fp16(q*s + b), activations fp16, fp32 sums, bf16 output.
 //
@@ -28,8 +29,8 @@
 //
 // Measured for QKV 5120 -> 10240 with the gate/up pair 5120 -> 2 x 17408, and
 // down 17408 -> 5120 (us; the GEMM's tiles before): 17 rows 50 + 27 (153 + 90),
-// 77 rows 64 + 34 (150 + 96), 160 rows 120 + 52 (152 + 99), 256 rows 177 + 68
-// (160 + 102).  What bounds it at 77 rows, by taking one part out: the
+// 77 rows 64 + 34 (150 + 96), 160 rows 120 + 52 (152 + 99), 300 rows 236 + 89
+// (272 + 127).  What bounds it at 77 rows, by taking one part out: the
 // dequantisation 5 us, the W loads 7, the X loads 10, the scale loads 4; the
 // products alone are 28 us at the clock that random operands leave.  Three
 // waves a SIMD (at most 168 registers) hide the rest better than two: 4 x 2
@@ -451,6 +452,16 @@ RowsPlan rows_plan(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const 
   return p;
 }
 
+// The plan's time (median error 5 % over the calls that q4_gemm_us names).
+double rows_us(const RowsPlan& p, uint32_t K, uint32_t cus) {
+  const uint32_t units = (K / 64 + kUnitGroups - 1) / kUnitGroups, wgs = p.tiles * p.slices;
+  const double work = (units + p.slices - 1) / p.slices * (p.mb == 1 ? 2.8 : p.mb == 2 ? 3.7 : 5.1);
+  auto round = [&](double n) { return work * (0.81 + 0.19 * wave_fill(n, cus)) + 7.4; };
+  double us = 6.7 + wgs / cus * round(cus);
+  if (wgs % cus) us += round(wgs % cus);
+  return p.slices > 1 ? us + 0.6 + 0.003 * wgs * p.mb : us;
+}
+
 template <int MB>
 void launch_rows(const RowsArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(q4_rows_kernel<MB>, dim3(a.tiles * a.slices), dim3(64 * WN * WK), 0, st, a);
@@ -462,14 +473,20 @@ void launch_rows(const RowsArgs& a, hipStream_t st) {
 bool q4_rows_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune) {
   // A forced GEMM plan is for the GEMM.
   if (M <= 16 || K % (64 * WK) != 0 || tune.rows_max <= 16 || tune.gemm_splits > 0 || tune.gemm_q > 0) return false;
-  // Up to 384 rows (at 300 rows of the sizes above 232 + 85 us against the
-  // GEMM's 275 + 126, at 512 345 + 128 against 293 + 134), and beyond while the
-  // tiles run in one round of the CUs (4096 -> 4096 at 512 rows: 46 against 57).
-  if (M <= (uint32_t)tune.rows_max) return true;
+  if (M <= (uint32_t)tune.rows_max && tune.rows_slices > 0) return true;
+  // While the tiles run in one round of the CUs, whatever the rows (4096 -> 4096
+  // at 512 rows: 46 us against the GEMM's 57).
+  const RowsPlan p = rows_plan(jobs, n_jobs, K, M, tune);
   const uint32_t cus = tune.cus > 0 ? (uint32_t)tune.cus : 256;
-  uint64_t tiles = 0;
-  for (int i = 0; i < n_jobs; ++i) tiles += job_tiles(jobs[i]);
-  return tiles * ((M + 32 * kMaxBlocks - 1) / (32 * kMaxBlocks)) <= cus;
+  if (p.tiles <= cus) return true;
+  if (M > (uint32_t)tune.rows_max) return false;
+  // Past that the tiles cross a round at other rows than the GEMM's (5120 -> 2 x
+  // 17408: 108 us against 151 at 192 rows, 165 against 151 at 256, 167 against
+  // 214 at 288; 1024 -> 65536: 45 each at 128, 80 against 46 at 224), so the
+  // estimates decide.  A tenth in this kernel's favour is the best line over the
+  // calls that q4_gemm_us names: up to 384 rows on average 0.1 % above the
+  // faster of the two (2.4 % with this kernel always).
+  return rows_us(p, K, cus) <= 1.1 * q4_gemm_us(jobs, n_jobs, K, M, tune);
 }
 
 void q4_rows_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune,

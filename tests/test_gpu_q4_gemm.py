@@ -295,3 +295,33 @@ def test_short_prompt_limits(rt, torch_dev, M, N, K):
     xb = synth.bf16_normal(rng, (M, K))
     (got,) = _project(rt, torch_dev, [mat], xb, M)
     assert_bf16_close(got, oracle.q4_project(xb, *mat), what=f"M{M} N{N} K{K}")
+
+
+@pytest.mark.parametrize("M,N,pair,K,gemm", [
+    (200, 65536, False, 512, True), (100, 12288, False, 512, False),  # several rounds of tiles, and one
+    (240, 16384, True, 768, True), (96, 16384, True, 768, False),
+])
+def test_short_prompt_route(torch_dev, M, N, pair, K, gemm):
+    """Up to 384 rows the faster of the short-prompt kernel and the GEMM takes
+    the call: the default's bits are that kernel's (their sums have different
+    orders) and within the bar of the oracle."""
+    import qm38
+    rng = np.random.default_rng(M + N)
+    mats = [synth.q4_matrix(rng, N, K) for _ in range(2 if pair else 1)]
+    dev = [_upload(torch_dev, *m) for m in mats]
+    jobs = [qm38.Runtime.job(*d, N) for d in dev]
+    xb = synth.bf16_normal(rng, (M, K))
+    xd = to_dev(xb, torch_dev)
+    got = {}
+    for name, env in (("default", {}), ("gemm", {"QM38_Q4_ROWS_MAX": 0}), ("rows", {"QM38_Q4_ROWS_SLICES": 1})):
+        with tuned(**env) as rt:
+            y = empty_bf16((M, N), torch_dev)
+            rt.q4_project_set(jobs[:1], [jobs[1] if pair else None], xd, K, M, [y])
+            got[name] = bf16_dev_to_f32(y)
+    rows = [0, M // 2, M - 1]
+    ref = oracle.q4_project(xb[rows], *mats[0])
+    if pair:
+        ref = oracle.swiglu(ref, oracle.q4_project(xb[rows], *mats[1]))
+    assert_bf16_close(got["default"][rows], ref, what=f"M{M} N{N} K{K}")
+    assert not np.array_equal(got["gemm"], got["rows"])
+    assert np.array_equal(got["default"], got["gemm" if gemm else "rows"])
