@@ -185,8 +185,9 @@ qm_status qm_q4_project(qm_runtime* rt, const qm_q4_job* jobs, int n_jobs,
  * is one launch that reads x once (the reference's mapped batch, whose jobs
  * would be a QKV projection and the pair kernels' gate/up, metal_runtime.rs:
  * 3599 with qwen38.metal:1404..3643); so are two rows, M > 16 (one GEMM
- * launch over plain and pair tiles) and large sets at M = 3..16.  Small sets
- * there run the plain jobs together and each pair as qm_q4_swiglu does.
+ * launch over plain and pair tiles), M = 3 and 4, and larger sets at M = 5..16
+ * where that is the faster.  The others run the plain jobs together and each
+ * pair as qm_q4_swiglu does.
  * n_jobs <= 8. */
 qm_status qm_q4_project_set(qm_runtime* rt, const qm_q4_job* jobs, const qm_q4_job* const* ups, int n_jobs,
                             const uint16_t* x, uint32_t in_elems, uint32_t M, uint16_t* const* outputs);

@@ -133,8 +133,8 @@ inline double wave_fill(double wgs, double cus) {
 hipError_t launch_q4_gemm(const Q4Job* jobs, int n_jobs, bool swiglu, const uint16_t* x,
                           uint32_t K, uint32_t M, const Workspace& ws, hipStream_t stream);
 
-// Q4 projection of QM38_Q4_LANES_LO .. 16 rows (q4_lanes.hip) of large matrices,
-// K a multiple of 256, bf16 outputs.  Jobs may mix plain projections and gate/up pairs.
+// Q4 projection of QM38_Q4_LANES_LO .. 16 rows (q4_lanes.hip) where it is the
+// faster, K a multiple of 256, bf16 outputs.  Jobs may mix plain projections and gate/up pairs.
 bool q4_lanes_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune);
 void q4_lanes_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, const Tuning& tune, size_t* partial_bytes);
 hipError_t launch_q4_lanes(const Q4Job* jobs, int n_jobs, const uint16_t* x, uint32_t K, uint32_t M,

@@ -335,27 +335,67 @@ LanesPlan lanes_plan(const Q4Job* jobs, int n_jobs, uint32_t K, const Tuning& tu
   return p;
 }
 
+// The plan's time, and what the call takes on the other kernels of these rows
+// (one MFMA streaming launch, or the decode kernel's: the plain jobs together
+// and each pair).  Fitted to 926 calls of 130 shapes (K 512 .. 17408, 16 .. 1444
+// tiles): median error 3 %, and 9 and 6 % of the others'.
+double lanes_us(const LanesPlan& p, uint32_t K, uint32_t M, uint32_t cus) {
+  const uint32_t units = (K / 64 + kUnitGroups - 1) / kUnitGroups, wgs = p.tiles * p.slices;
+  const double work = (units + p.slices - 1) / p.slices * 2.6 * (1.0 + 0.0044 * M);
+  auto round = [&](uint32_t n) { return work * (0.72 + 0.28 * n / cus) + 4.6; };
+  double us = 1.7 + wgs / cus * round(cus);
+  if (wgs % cus) us += round(wgs % cus);
+  return p.slices > 1 ? us + 3.3 + 0.0032 * wgs : us;
+}
+
+struct Others {
+  double us;
+  int launches;
+};
+Others others_us(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune) {
+  double mb = 0.0;  // weights and tables
+  int pairs = 0;
+  for (int i = 0; i < n_jobs; ++i) {
+    const bool pair = jobs[i].mode == kQ4OutSwiglu;
+    mb += (double)jobs[i].rows * (pair ? 2 : 1) * K * 0.5625e-6;
+    pairs += pair;
+  }
+  if (tune.q4_mma_lo > 0 && (int)M >= tune.q4_mma_lo && (int)M <= tune.q4_mma_hi)
+    return {6.9 + mb / (pairs ? 3.9 : 4.28), 1};
+  const bool long_k = tune.q4_mma_k > 0 && K > (uint32_t)tune.q4_mma_k;
+  if (long_k && M <= 8) return {24.0 + mb / 3.6, 1};
+  const int launches = pairs + (pairs < n_jobs);
+  const double rate = (5.1 - 0.105 * M) / (long_k ? 1.49 - 0.03 * ((int)M - 8) : 1.0);
+  return {5.6 + 5.1 * (launches - 1) + mb / rate, launches};
+}
+
 }  // namespace
 
 bool q4_lanes_supported(const Q4Job* jobs, int n_jobs, uint32_t K, uint32_t M, const Tuning& tune) {
   if (M < (uint32_t)tune.lanes_lo || M > 16 || tune.lanes_lo <= 0 || K % (64 * WK) != 0) return false;
   // A forced plan of another kernel is for that kernel.
   if (tune.q4_nt > 0 || tune.q4_rpw > 0 || tune.q4_split > 0 || tune.q4_mma_c > 0 || !tune.q4_stream) return false;
-  uint64_t tiles = 0;
-  for (int i = 0; i < n_jobs; ++i) {
+  for (int i = 0; i < n_jobs; ++i)
     if (jobs[i].mode != kQ4OutBf16 && jobs[i].mode != kQ4OutSwiglu) return false;
-    tiles += job_tiles(jobs[i]);
-  }
   if (tune.lanes_slices > 0) return true;
-  // Where the tiles fill half of the CUs without K slices (the set above).
+  const LanesPlan p = lanes_plan(jobs, n_jobs, K, tune);
+  const uint64_t cus = tune.cus > 0 ? (uint64_t)tune.cus : 256;
+  const Others o = others_us(jobs, n_jobs, K, M, tune);
+  // Where the tiles fill half of the CUs the estimates decide: a tile more than
+  // a round's costs a round (5120 -> 192 rows a tile at 9 rows: 35 us for 256
+  // tiles and 58 for 257, where the decode kernel takes 37 and 38; at 16 rows 37
+  // and 60 against 44 and 47), and 5 to 9 rows of a round two thirds full lose
+  // too (160 tiles 31 us against 25 .. 27).  On 926 timed calls of 130 shapes the
+  // choice is on average 1.7 % above the faster kernel (16.9 with this one always).
+  if (2 * (uint64_t)p.tiles >= cus) return lanes_us(p, K, M, (uint32_t)cus) <= 1.05 * o.us;
   // Smaller matrices need slices and their second launch, and the kernels that
   // cut finer stay ahead (4096 -> 4096: 6 .. 9 us against 11; QKV alone 13 .. 15
   // against 16 up to 9 rows) until the decode kernel's time grows with the rows:
-  // QKV 17.4 us at 12 rows; down 17408 -> 5120 27 us at 9 rows and 37 at 16,
-  // 19.5 here (up to 8 rows the MFMA streaming kernel takes it in 16 .. 19).
-  const uint64_t cus = tune.cus > 0 ? (uint64_t)tune.cus : 256;
-  if (2 * tiles >= cus) return true;
-  return (M >= 9 && K > 8192 && 16 * tiles >= cus) || (M >= 12 && 5 * tiles >= cus);
+  // QKV 17.2 us against 20.0 at 16; down 17408 -> 5120 28 us at 9 rows and 38 at
+  // 16, 21 here (up to 8 rows the MFMA streaming kernel takes it in 17 .. 20).
+  // One launch of narrow rows stays there (2560 -> 15674 at 12 rows 13 us, 15 here).
+  return (M >= 9 && K > 8192 && 16 * (uint64_t)p.tiles >= cus) ||
+         (M >= 12 && (K > 3072 || o.launches > 1) && 5 * (uint64_t)p.tiles >= cus);
 }
 
 void q4_lanes_workspace(const Q4Job* jobs, int n_jobs, uint32_t K, const Tuning& tune, size_t* partial_bytes) {

@@ -518,3 +518,33 @@ def test_large_sets_of_a_few_rows(rt, torch_dev, M):
     y, h = (bf16_dev_to_f32(o) for o in outs)
     assert_bf16_close(y, oracle.q4_project(xb, *mats[0]), what="plain")
     assert_bf16_close(h, oracle.swiglu(oracle.q4_project(xb, *mats[1]), oracle.q4_project(xb, *mats[2])), what="pair")
+
+
+@pytest.mark.parametrize("M,tiles,pair,lanes", [(16, 236, False, True), (8, 257, False, False), (16, 257, True, False),
+                                                (4, 250, True, True)])
+def test_lanes_route(torch_dev, M, tiles, pair, lanes):
+    """A round of 192-row tiles goes to q4_lanes_kernel, a tile more does not:
+    the default's bits are those of the forced or excluded kernel (their sums
+    have different orders), and both lie within the bar of the oracle."""
+    import qm38
+    rng = np.random.default_rng(M + tiles)
+    K, N = 1024, tiles * (96 if pair else 192) - 5
+    mats = [synth.q4_matrix(rng, N, K) for _ in range(2 if pair else 1)]
+    jobs = [qm38.Runtime.job(*(to_dev(a, torch_dev) for a in m), N) for m in mats]
+    xb = synth.bf16_normal(rng, (M, K))
+    xd = to_dev(xb, torch_dev)
+    got = {}
+    for name, env in (("default", {}), ("lanes", {"QM38_Q4_LANES_SLICES": 1}), ("sliced", {"QM38_Q4_LANES_SLICES": 2}),
+                      ("others", {"QM38_Q4_LANES_LO": 0})):
+        with tuned(**env) as rt:
+            y = empty_bf16((M, N), torch_dev)
+            rt.q4_project_set(jobs[:1], [jobs[1] if pair else None], xd, K, M, [y])
+            got[name] = bf16_dev_to_f32(y)
+    rows = [0, M - 1]
+    ref = oracle.q4_project(xb[rows], *mats[0])
+    if pair:
+        ref = oracle.swiglu(ref, oracle.q4_project(xb[rows], *mats[1]))
+    for name, y in got.items():
+        assert_bf16_close(y[rows], ref, what=f"{name} M {M} tiles {tiles}")
+    assert not np.array_equal(got["lanes"], got["others"])
+    assert np.array_equal(got["default"], got["lanes" if lanes else "others"])
