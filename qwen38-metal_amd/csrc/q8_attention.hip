@@ -791,11 +791,7 @@ __global__ __launch_bounds__(64) void q8_combine_small_kernel(AttnArgs args) {
   }
 }
 
-// Four outputs as bf16, and with the sigmoid of four bf16 gates.  The gate
-// takes v_exp_f32 and v_rcp_f32 (within an ulp each; the error of the product
-// -v log2(e) grows with |v| and stays below 2^-16 of the result for every gate
-// whose sigmoid is above 1e-30, against the 2^-9 of the bf16 store): the
-// library forms took longer than a tile's softmax.
+// Four outputs as bf16, and with the sigmoid of four bf16 gates.
 __device__ __forceinline__ u32x2 bf16x4_of(floatx4 v) {
   return u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
                (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
@@ -805,7 +801,7 @@ __device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
   for (int i = 0; i < 4; ++i) {
     const uint32_t w = i < 2 ? gate.x : gate.y;
     const float x = i & 1 ? bf16_hi_f32(w) : bf16_lo_f32(w);
-    v[i] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * x));
+    v[i] *= sigmoid_f(x);
   }
   return bf16x4_of(v);
 }
