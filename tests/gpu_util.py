@@ -16,6 +16,16 @@ def to_dev(a: np.ndarray, dev):
     return torch.from_numpy(a).to(dev)
 
 
+def off_by_8(a: np.ndarray, dev):
+    """`a` on the device at an address that is 8, but not 16 bytes aligned."""
+    import torch
+    n = 8 // a.dtype.itemsize
+    flat = to_dev(np.concatenate([np.zeros(n, a.dtype), a.reshape(-1)]), dev)
+    t = flat[n:].reshape(a.shape)
+    assert t.data_ptr() % 16 == 8
+    return t
+
+
 def from_dev(t, dtype=None) -> np.ndarray:
     import torch
     torch.cuda.synchronize()

@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_util import assert_bf16_close, bf16_dev_to_f32, empty_bf16, to_dev, tuned
+from gpu_util import assert_bf16_close, bf16_dev_to_f32, empty_bf16, off_by_8, to_dev, tuned
 from qm38 import QmError, synth
 
 pytestmark = pytest.mark.gpu
@@ -548,3 +548,26 @@ def test_lanes_route(torch_dev, M, tiles, pair, lanes):
         assert_bf16_close(y[rows], ref, what=f"{name} M {M} tiles {tiles}")
     assert not np.array_equal(got["lanes"], got["others"])
     assert np.array_equal(got["default"], got["lanes" if lanes else "others"])
+
+
+@pytest.mark.parametrize("M", [3, 16])
+def test_lanes_kernel_on_8_byte_aligned_tables(torch_dev, M):
+    # Weights, scales and biases need 8-byte alignment only; the kernel's DMAs
+    # take 16 bytes.  K 768: scale rows of 24 bytes.
+    import qm38
+    rng = np.random.default_rng(M)
+    K, N = 768, 200
+    mats = [synth.q4_matrix(rng, N, K) for _ in range(3)]
+    xb = synth.bf16_normal(rng, (M, K))
+    xd = to_dev(xb, torch_dev)
+    runs = []
+    with tuned(QM38_Q4_LANES_SLICES=2) as rt:
+        for put in (to_dev, off_by_8):
+            j, g, u = (qm38.Runtime.job(*(put(a, torch_dev) for a in m), N) for m in mats)
+            outs = [empty_bf16((M, N), torch_dev) for _ in range(2)]
+            rt.q4_project_set([j, g], [None, u], xd, K, M, outs)
+            runs.append([bf16_dev_to_f32(o) for o in outs])
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+    assert_bf16_close(runs[0][0], oracle.q4_project(xb, *mats[0]))
+    assert_bf16_close(runs[0][1], oracle.swiglu(*(oracle.q4_project(xb, *m) for m in mats[1:])))

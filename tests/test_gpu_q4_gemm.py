@@ -1,11 +1,12 @@
-"""GPU parity of the Q4 prefill GEMM (M > 16) against the CPU oracle.
+"""GPU parity of the Q4 prefill kernels (M > 16) against the CPU oracle.
 
 Ports mapped_q4_matmul_batch_matches_each_prompt_row (metal_runtime.rs:9766),
 simdgroup_q4_matmul_batch_matches_cpu_reference (:10560),
 wide_simdgroup_q4_matmul_batch_matches_cpu_reference (:10620) and
 fused_q4_mlp_batch_matches_cpu_reference at M = 256 (:10726), plus the
-BASELINE prefill shapes.  The kernel computes like the reference's prefill
-path: fp16(q*s + b) weights, fp16 activations, fp32 accumulation; the
+BASELINE prefill shapes.  Small sizes run on the short-prompt kernel by
+default, so every test that takes a runtime runs on the default route and on
+the GEMM alone.  Both kernels compute like the reference's prefill path: fp16(q*s + b) weights, fp16 activations, fp32 accumulation; the
 oracle is exact (fp64).  Bar: bf16 outputs within 1e-4 of max|ref| beyond
 the bf16 output rounding (tests/gpu_util.py).
 """
@@ -15,10 +16,16 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_util import assert_bf16_close, bf16_dev_to_f32, empty_bf16, to_dev, tuned
+from gpu_util import assert_bf16_close, bf16_dev_to_f32, empty_bf16, off_by_8, to_dev, tuned
 from qm38 import synth
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=["default", "gemm"])
+def rt(request, torch_dev):
+    with tuned(QM38_Q4_ROWS_MAX=0 if request.param == "gemm" else None) as r:
+        yield r
 
 
 def _upload(dev, packed, s, b):
@@ -100,7 +107,7 @@ def test_constant_nibble_closed_form(rt, torch_dev):
 
 
 def test_activation_beyond_fp16_range_saturates(rt, torch_dev):
-    # The GEMM stages activations in fp16; a bf16 value beyond +-65504 is
+    # Both kernels take activations as fp16; a bf16 value beyond +-65504 is
     # clamped to +-65504 instead of becoming an infinity, so the result equals
     # the exact projection of the clamped input and every output stays finite.
     rng = np.random.default_rng(21)
@@ -179,9 +186,10 @@ def test_prefill_27b_shapes(rt, torch_dev, M):
 
 @pytest.mark.parametrize("M", [33, 300])
 def test_split_k_swiglu_and_determinism(rt, torch_dev, M):
-    # K = 2048 (32 groups) with few output tiles: the launch splits K across
-    # workgroups, and the last slice of each tile adds the slices in a fixed
-    # order, so two calls agree bit for bit.
+    # K = 2048 (32 groups) with few output tiles: both kernels split K across
+    # workgroups and add the slices of a tile in a fixed order (the GEMM in its
+    # last slice, the short-prompt kernel in a second launch), so two calls
+    # agree bit for bit.
     import qm38
     rng = np.random.default_rng(90 + M)
     K, I = 2048, 384
@@ -232,11 +240,11 @@ def test_worker_step_ranges(torch_dev, knob, q):
 
 
 @pytest.mark.parametrize("M", [40, 300])
-@pytest.mark.parametrize("knob", [None, ("QM38_GEMM_SPLITS", 3), ("QM38_GEMM_Q", 21)])
+@pytest.mark.parametrize("knob", [None, ("QM38_Q4_ROWS_MAX", 0), ("QM38_GEMM_SPLITS", 3), ("QM38_GEMM_Q", 21)])
 def test_mixed_set_in_one_launch(torch_dev, M, knob):
     """qm_q4_project_set with prefill rows: plain projections (256-row tiles)
-    and SwiGLU pairs (128 gate + 128 up rows per tile) in one GEMM launch,
-    whole tiles, K split into slices, and stream-K ranges that cut tiles of
+    and SwiGLU pairs (128 gate + 128 up rows per tile) in one launch of the
+    short-prompt kernel and of the GEMM: whole tiles, K split into slices, and stream-K ranges that cut tiles of
     both kinds; every output within the bar of the oracle."""
     import qm38
     env = {} if knob is None else {knob[0]: knob[1]}
@@ -257,11 +265,13 @@ def test_mixed_set_in_one_launch(torch_dev, M, knob):
 
 
 @pytest.mark.parametrize("M", [17, 32, 33, 65, 96, 97, 200])
-@pytest.mark.parametrize("K,slices", [(256, None), (512, 2), (1280, 1), (2304, 5), (4352, None)])
+@pytest.mark.parametrize("K,slices", [(256, None), (512, 2), (1280, 1), (2304, 5), (4352, None), (2304, 2), (4352, 3),
+                                      (4352, 4)])
 def test_short_prompt_kernel(torch_dev, M, K, slices):
-    """17..384 rows with K a multiple of 256 (q4_rows_kernel): one to three row
+    """q4_rows_kernel (17 rows and more, K a multiple of 256): one to three row
     blocks a tile and several row tiles, rows and weight rows that end inside a
-    block, K units (512) cut short, K slices even and uneven, plain jobs and
+    block, K units (512) cut short, K slices of one unit and of several that start at
+    even and odd ones, plain jobs and
     pairs in one launch; within the bar of the oracle and the same bits twice."""
     import qm38
     with tuned(QM38_Q4_ROWS_SLICES=slices) as rt:
@@ -325,3 +335,20 @@ def test_short_prompt_route(torch_dev, M, N, pair, K, gemm):
     assert_bf16_close(got["default"][rows], ref, what=f"M{M} N{N} K{K}")
     assert not np.array_equal(got["gemm"], got["rows"])
     assert np.array_equal(got["default"], got["gemm" if gemm else "rows"])
+
+
+def test_short_prompt_kernel_on_8_byte_aligned_tables(torch_dev):
+    # Weights, scales and biases need 8-byte alignment only; the kernel's DMAs
+    # take 16 bytes.
+    import qm38
+    rng = np.random.default_rng(15)
+    N, K, M = 200, 768, 40
+    mat = synth.q4_matrix(rng, N, K)
+    xb = synth.bf16_normal(rng, (M, K))
+    with tuned(QM38_Q4_ROWS_SLICES=2) as rt:
+        (want,) = _project(rt, torch_dev, [mat], xb, M)
+        odd = [off_by_8(a, torch_dev) for a in mat]
+        y = empty_bf16((M, N), torch_dev)
+        rt.q4_project([qm38.Runtime.job(*odd, N)], to_dev(xb, torch_dev), K, M, [y])
+        assert np.array_equal(bf16_dev_to_f32(y), want)
+    assert_bf16_close(want, oracle.q4_project(xb, *mat))
