@@ -68,6 +68,7 @@ qm_status qm::order_workspaces(qm_runtime* rt) {
   // A captured use runs when its graph does; the caller orders that.
   if (rt->device < 0 || stream_capturing(rt->stream)) return QM_OK;
   if (rt->ws_sync) {
+    DeviceGuard g(rt->device);
     const hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return hip_check(e, "workspace order");
     rt->ws_sync = rt->ws_wait = false;
