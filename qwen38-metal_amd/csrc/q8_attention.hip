@@ -822,11 +822,11 @@ __device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
 // Few rows leave the chip idle if one workgroup walks all tiles (5 rows of
 // 24 / 4 heads on 20001 tokens ran on 4 workgroups, 1570 us), so the tiles
 // are then split over args.splits workgroups, whose (O, m, l) the combine
-// kernel merges (33 us with the merge).
+// kernel merges (36 us with the merge).
 //
 // What bounds it: at 2048 rows on 4096 tokens (64 / 8 heads of 128) about 220
 // VALU operations and 24 MFMAs (768 cycles) per wave and tile, two waves per
-// SIMD; 505 us, 680 TFLOP/s.  The 16-wide kernel before it (one page a step,
+// SIMD; 531 us, 647 TFLOP/s, of which the gate's exponential and division 10.  The 16-wide kernel before it (one page a step,
 // columns padded to the group size, the maximum exchanged every page) took
 // 870 us.
 template <int D, int W>
