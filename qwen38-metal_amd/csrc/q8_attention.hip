@@ -791,17 +791,33 @@ __global__ __launch_bounds__(64) void q8_combine_small_kernel(AttnArgs args) {
   }
 }
 
+// Sigmoid of a bf16 gate.  A bf16 (8 bits) times log2(e) cut to 16 bits is exact,
+// and what the cut takes from the exponential goes into the Newton step of the
+// reciprocal.  Over every bf16 gate from -87 up: at most 1.95 ulp, 0.250 rms,
+// where expf and an IEEE division (sigmoid_f) have 1.98 and 0.252; a sigmoid
+// below the smallest normal number is zero.  The limits, which pass NaN on,
+// keep infinities out of the products.  A wave ends with up to 128 of these in
+// a row, and a short prompt waits for that: 2 rows of 24 / 4 heads of 256 take
+// 17.2 us a call, 23.6 with sigmoid_f and the integer form of f32_to_bf16.
+__device__ __forceinline__ float gate_sigmoid(float x) {
+  constexpr float kCut = 1.44268798828125f;
+  constexpr float kRest = (float)((1.0 - 1.4426950408889634 / kCut) * 0.6931471805599453);
+  const float t = __builtin_elementwise_maximum(__builtin_elementwise_minimum(x * -kCut, 127.0f), -126.0f);
+  const float e = __builtin_amdgcn_exp2f(t), d = 1.0f + e, q = __builtin_amdgcn_rcpf(d);
+  const float n = __builtin_fmaf(e * (t * kRest), q, __builtin_fmaf(-d, q, 1.0f));
+  return __builtin_fmaf(n, q, q);
+}
+
 // Four outputs as bf16, and with the sigmoid of four bf16 gates.
 __device__ __forceinline__ u32x2 bf16x4_of(floatx4 v) {
-  return u32x2{(uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
-               (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16)};
+  return u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
 }
 __device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t w = i < 2 ? gate.x : gate.y;
     const float x = i & 1 ? bf16_hi_f32(w) : bf16_lo_f32(w);
-    v[i] *= sigmoid_f(x);
+    v[i] *= gate_sigmoid(x);
   }
   return bf16x4_of(v);
 }
@@ -1166,7 +1182,7 @@ __global__ __launch_bounds__(64 * W, attn_prefill_waves(D, W)) void q8_prefill_k
         const uint32_t d = 32 * db + 8 * (e >> 2) + 4 * hf + (e & 3);
         if (d >= dr) continue;
         float v = o[db][e] * inv;
-        if (args.gate) v *= sigmoid_f(bf16_to_f32(args.gate[obase + d]));
+        if (args.gate) v *= gate_sigmoid(bf16_to_f32(args.gate[obase + d]));
         args.o[obase + d] = f32_to_bf16(v);
       }
   }
@@ -1214,7 +1230,7 @@ __global__ __launch_bounds__(256) void q8_combine_rows_kernel(AttnArgs args) {
   } else {
     for (int e = 0; e < 4 && d0 + e < dr; ++e) {
       float v = acc[e];
-      if (args.gate) v *= sigmoid_f(bf16_to_f32(args.gate[oi + e]));
+      if (args.gate) v *= gate_sigmoid(bf16_to_f32(args.gate[oi + e]));
       args.o[oi + e] = f32_to_bf16(v);
     }
   }

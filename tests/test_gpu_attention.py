@@ -338,6 +338,43 @@ def test_prefill_launch_shapes(rt, torch_dev, D, H, KVH, waves, splits):
     _check_cache(cache, mirror)
 
 
+@pytest.mark.parametrize("D,M,start", [(128, 5, 20), (256, 5, 20), (128, 6, 1300)])
+def test_prefill_gate_range(rt, torch_dev, D, M, start):
+    """Gates of any size in the unsplit epilogue and in the merge: exactly open
+    and shut ones, infinities, and sigmoids far below the others'; the store
+    with and without 8-byte alignment gives the same bits, and a NaN gate NaN."""
+    H, KVH = 16, 2
+    rng = np.random.default_rng(D + M)
+    cache, mirror = rt.create_q8_kv_state(KVH, D, start + M), Mirror(KVH, D)
+    _fill(rt, torch_dev, cache, mirror, rng, start, H, KVH, D)
+    q_bits, q_f, _g, _gf, k, v = _rand_qkv(rng, M, H, KVH, D)
+    mirror.append(k, v)
+    special = np.array([0.0, -0.0, 1e-30, 64.0, -30.0, -60.0, -80.0, -87.0, 88.0, 1e4, -1e4, 3e38, -3e38, np.inf, -np.inf],
+                       np.float32)
+    g = rng.standard_normal((M, H, D)).astype(np.float32) * 8
+    pick = rng.random(g.shape) < 0.5
+    g[pick] = rng.choice(special, int(pick.sum()))
+    g_bits = synth.f32_to_bf16(g)
+    ref = mirror.reference(q_f, synth.bf16_to_f32(g_bits), start)
+    got = _prefill(rt, torch_dev, cache, q_bits, g_bits, k, v, H)
+    assert_bf16_close(got, ref, what="gates")
+    shut = synth.bf16_to_f32(g_bits) < -1e3
+    assert np.all(got[shut] == 0.0)
+    # Relative to the value itself: sigmoids of any size are as exact as the rest.
+    open_ref = mirror.reference(q_f, None, start)
+    far = (np.abs(synth.bf16_to_f32(g_bits)) <= 87.0) & (np.abs(open_ref) > 1e-2 * np.abs(open_ref).max())
+    assert np.all(np.abs(got[far] - ref[far]) <= (2.0 ** -8 + 2e-2) * np.abs(ref[far]) + 1e-38)
+    cache.truncate(start)
+    flat = empty_bf16((M * H * D + 1,), torch_dev)
+    rt.gqa_attention_q8_prefill(cache, to_dev(q_bits, torch_dev), to_dev(g_bits, torch_dev), to_dev(k, torch_dev),
+                                to_dev(v, torch_dev), H, M, flat.data_ptr() + 2)
+    assert np.array_equal(bf16_dev_to_f32(flat[1:]).reshape(M, H, D), got)
+    cache.truncate(start)
+    g_bits[M - 1, 3, 7] = 0x7FC0
+    out = _prefill(rt, torch_dev, cache, q_bits, g_bits, k, v, H)
+    assert np.isnan(out[M - 1, 3, 7]) and np.isnan(out).sum() == 1
+
+
 def test_prefill_on_two_streams_of_one_runtime(rt, torch_dev):
     """Split prefills that one runtime enqueues on five streams in turn: one set
     of partials, in stream order."""
