@@ -842,7 +842,7 @@ __device__ __forceinline__ u32x2 gated_bf16x4(floatx4 v, u32x2 gate) {
 //
 // What bounds it: at 2048 rows on 4096 tokens (64 / 8 heads of 128) about 220
 // VALU operations and 24 MFMAs (768 cycles) per wave and tile, two waves per
-// SIMD; 531 us, 647 TFLOP/s, of which the gate's exponential and division 10.  The 16-wide kernel before it (one page a step,
+// SIMD; 527 us, 652 TFLOP/s.  The 16-wide kernel before it (one page a step,
 // columns padded to the group size, the maximum exchanged every page) took
 // 870 us.
 template <int D, int W>

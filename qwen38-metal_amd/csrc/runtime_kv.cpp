@@ -299,10 +299,10 @@ qm_status plan_decode_chunk(qm_runtime* rt, qm_kv* const* seqs, uint32_t nb, Dec
 //
 // Waves.  Eight share an unpacked tile among 256 columns, four among 128.
 // Head storage of 256 leaves a 4-wave workgroup one wave per SIMD, so it takes
-// eight from 1024 columns on (24 / 4 heads, 300 rows on 4000 tokens: 80 us
-// against 97; 40 rows: 45 against 39).  Narrower heads take eight once those
+// eight from 1024 columns on (24 / 4 heads, 300 rows on 4000 tokens: 79 us
+// against 97; 40 rows: 46 against 39).  Narrower heads take eight once those
 // workgroups fill the chip twice (64 / 8 heads of 128, 2048 rows on 4096
-// tokens: 535 against 570 us; 1000 on 1000: 117 against 110).  Heads of 64 keep
+// tokens: 532 against 567 us; 1000 on 1000: 113 against 107).  Heads of 64 keep
 // four (8 heads, 2000 rows on 4000: 68 against 81 us).
 //
 // Splits.  One workgroup per column block fills the chip when the rows are
