@@ -124,3 +124,32 @@ def test_few_rows_capture_without_a_warm_call(torch_dev, M, specs, K):
                 assert_bf16_close(bf16_dev_to_f32(o), ref, what=f"replay {i}")
                 assert_bf16_close(bf16_dev_to_f32(r), ref, what=f"eager {i}")
                 o.fill_(-1)
+
+
+@pytest.mark.parametrize("M,N,K,env", [(40, 700, 4096, {"QM38_Q4_ROWS_SLICES": 4}), (300, 300, 2048, {"QM38_GEMM_SPLITS": 3}),
+                                       (3, 512, 9216, {})])
+def test_capture_after_a_warm_call_elsewhere(torch_dev, M, N, K, env):
+    """A call warmed on one stream may be captured on another (the stream that
+    is left has used a workspace), and the runtime goes on after it: every
+    replay, and eager calls between them, equal the call before the capture."""
+    import torch
+    rng = np.random.default_rng(M)
+    with tuned(**env) as rt:
+        mat = synth.q4_matrix(rng, N, K)
+        job = _job(mat, torch_dev)
+        x = to_dev(synth.bf16_normal(rng, (M, K)), torch_dev)
+        want, got, eager = (empty_bf16((M, N), torch_dev) for _ in range(3))
+        rt.q4_project([job], x, K, M, [want])
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            rt.set_stream(torch.cuda.current_stream())
+            rt.q4_project([job], x, K, M, [got])
+        rt.set_stream(torch.cuda.current_stream())
+        for _ in range(3):
+            got.fill_(-1)
+            eager.fill_(-1)
+            graph.replay()
+            rt.q4_project([job], x, K, M, [eager])
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(eager, want)
+    assert_bf16_close(bf16_dev_to_f32(want), oracle.q4_project(x.cpu().numpy().view(np.uint16), *mat))
